@@ -23,6 +23,11 @@ static_assert(CRVPT_KPN_PARAMS == kKpnParams, "parameter count of the C ABI");
 
 constexpr size_t kFragBytes = size_t(kKpnLayers) * 9 * 2 * 64 * 16;  // bf16x8 fragments of all layers
 
+// Persistent convolution workgroups per CU: the two that fit (148 vector registers and 32 accumulators per lane), so that
+// every tile after a workgroup's first has its halo prefetched and the weights are read once (1920x1080 inference with
+// 1 / 2 / 3 / 4 / 8 per CU: 628 / 569 / 614 / 572 / 597 us).
+constexpr int kConvBlocksPerCU = 2;
+
 struct KpnModel {
     DevBuf params, grads, m1, m2, wFwd, wBwd, loss;
     DevBuf act, logits, dzA, dzB, pred, gradWork;
@@ -111,13 +116,13 @@ int forward(const float* features, int n, int h, int w, hipStream_t s) {
     KpnModel& k = *g_kpn;
     const size_t P = size_t(n) * h * w;
     if (int rc = ensureActivations(P)) return rc;
-    const int blocks = k.cuCount * 8;
+    const int blocks = k.cuCount * kConvBlocksPerCU;
     HIP_TRY(launchKpnPack(features, actOf(k, 0, P), n, h, w, s));
     for (int l = 0; l < kKpnLayers - 1; l++)
         HIP_TRY(launchKpnConv(0, actOf(k, l, P), fragOf(k.wFwd, l), biasOf(k, l), nullptr, actOf(k, l + 1, P), n, h,
-                              w, 0, blocks, s));
+                              w, blocks, s));
     HIP_TRY(launchKpnConv(1, actOf(k, kKpnLayers - 1, P), fragOf(k.wFwd, kKpnLayers - 1),
-                          biasOf(k, kKpnLayers - 1), nullptr, k.logits.ptr, n, h, w, 0, blocks, s));
+                          biasOf(k, kKpnLayers - 1), nullptr, k.logits.ptr, n, h, w, blocks, s));
     return CRVPT_OK;
 }
 
@@ -202,8 +207,8 @@ int crvpt_kpn_compute_gradients(const float* features, const float* noisy, const
                                     n, h, w, blocks, k.gradWork.as<float>(), s));
         if (l > 0) {
             // gradient of the layer's input, through the ReLU that produced it
-            HIP_TRY(launchKpnConv(2, dz, fragOf(k.wBwd, l), nullptr, actOf(k, l, P), dzNext, n, h, w, 1,
-                                  k.cuCount * 8, s));
+            HIP_TRY(launchKpnConv(2, dz, fragOf(k.wBwd, l), nullptr, actOf(k, l, P), dzNext, n, h, w,
+                                  k.cuCount * kConvBlocksPerCU, s));
             std::swap(dz, dzNext);
         }
     }

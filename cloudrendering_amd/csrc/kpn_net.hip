@@ -35,17 +35,105 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Stages the (16 + 2)^2 input pixels around output tile (y0, x0) of image n into LDS (zero outside the image).
-__device__ __forceinline__ void stageHalo(__bf16* tile, const __bf16* __restrict__ in, int n, int H, int W, int y0,
-                                          int x0) {
-    for (int c = threadIdx.x; c < kHalo * kHalo * 4; c += blockDim.x) {
-        const int pix = c >> 2, ch = c & 3;
-        const int hy = pix / kHalo, hx = pix - hy * kHalo;
-        const int gy = y0 + hy - 1, gx = x0 + hx - 1;
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        if (gy >= 0 && gy < H && gx >= 0 && gx < W)
-            v = *reinterpret_cast<const uint4*>(in + ((size_t(n) * H + gy) * W + gx) * kC + ch * 8);
-        *reinterpret_cast<uint4*>(tile + pix * kPixStride + ch * 8) = v;
+// Tile index of a persistent workgroup's k-th tile. Workgroups go to the 8 XCDs round robin, each with its own L2:
+// XCD x takes the x-th eighth of the tiles, so that neighbouring tiles, which share their halo pixels, meet in one L2.
+constexpr int kXcds = 8;
+
+struct TileWalk {
+    int tilesX, tilesY, end, step, ti;
+    int n, y0, x0;
+    __device__ __forceinline__ TileWalk(int N, int H, int W) {
+        tilesX = (W + kTile - 1) / kTile;
+        tilesY = (H + kTile - 1) / kTile;
+        const int numTiles = N * tilesX * tilesY;
+        const int xcd = int(blockIdx.x) % kXcds, slot = int(blockIdx.x) / kXcds;
+        const int groups = min(int(gridDim.x), kXcds);  // XCDs that have a workgroup
+        const int begin = int(int64_t(numTiles) * xcd / groups);
+        end = int(int64_t(numTiles) * (xcd + 1) / groups);
+        step = (int(gridDim.x) - xcd + kXcds - 1) / kXcds;  // workgroups of this XCD
+        ti = begin + slot;
+        locate();
+    }
+    __device__ __forceinline__ void locate() {
+        n = ti / (tilesX * tilesY);
+        const int r = ti - n * tilesX * tilesY;
+        y0 = (r / tilesX) * kTile;
+        x0 = (r % tilesX) * kTile;
+    }
+    __device__ __forceinline__ bool valid() const { return ti < end; }
+    __device__ __forceinline__ void next() {
+        ti += step;
+        locate();
+    }
+};
+
+// The (16 + 2)^2 input pixels around output tile (y0, x0) of image n, zero outside the image: 1296 16-byte chunks, of
+// which thread t holds chunks t, t + 256, ... in registers between load() and store() into LDS. The next tile's halo
+// is loaded before the current tile is computed, so its latency is hidden behind the MFMAs and stores.
+constexpr int kHaloChunks = kHalo * kHalo * 4;
+constexpr int kHaloRegs = (kHaloChunks + 255) / 256;
+
+struct Halo {
+    uint4 v[kHaloRegs];
+    __device__ __forceinline__ void load(const __bf16* __restrict__ in, int n, int H, int W, int y0, int x0) {
+        const __bf16* img = in + size_t(n) * H * W * kC;
+#pragma unroll
+        for (int k = 0; k < kHaloRegs; k++) {
+            const int c = threadIdx.x + k * 256, pix = c >> 2, ch = c & 3;
+            const int hy = pix / kHalo, hx = pix - hy * kHalo;
+            const int gy = y0 + hy - 1, gx = x0 + hx - 1;
+            v[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (c < kHaloChunks && unsigned(gy) < unsigned(H) && unsigned(gx) < unsigned(W))
+                v[k] = *reinterpret_cast<const uint4*>(img + (size_t(gy) * W + gx) * kC + ch * 8);
+        }
+    }
+    __device__ __forceinline__ void store(__bf16* tile) const {
+#pragma unroll
+        for (int k = 0; k < kHaloRegs; k++) {
+            const int c = threadIdx.x + k * 256;
+            if (c < kHaloChunks) *reinterpret_cast<uint4*>(tile + (c >> 2) * kPixStride + (c & 3) * 8) = v[k];
+        }
+    }
+};
+
+// The nine taps of a 3x3 convolution for one wave: output rows wave * 4 .. + 3 of the staged tile, acc[row][N tile].
+// The MFMA takes the weights as its A operand and the pixels as B, so the 16x16 result is channels x pixels: lane
+// (m, kb) holds output channels nt * 16 + kb * 4 + 0..3 of pixel m of the tile row, four consecutive channels that
+// leave in one 8-byte (bf16) or 16-byte (f32) store. FLIP mirrors the taps (the backward data pass).
+//
+// Bound by LDS reads: a 1-KB pixel operand feeds two MFMAs, and at 128 B per cycle the four waves' reads would take as
+// long as their MFMAs. So each operand is read once and used by every output row it is a tap of (18 reads for 72
+// MFMAs instead of 36), in an order that keeps every accumulator's taps ascending: results are those of a plain loop
+// over the taps, bit for bit. FLIP is a template parameter because only then do the reads coincide at compile time.
+template <bool FLIP>
+__device__ __forceinline__ void convTaps(const __bf16* tile, const bf16x8 (&B)[9][2], int wave, int m, int kb,
+                                         f32x4 (&acc)[4][2]) {
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++) acc[mt][0] = acc[mt][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int r = 0; r < 6; r++) {
+        const int hy = FLIP ? 5 - r : r;  // staged row of the wave's six
+#pragma unroll
+        for (int kx = 0; kx < 3; kx++) {
+            const int hx = FLIP ? 2 - kx : kx;
+            const bf16x8 A =
+                *reinterpret_cast<const bf16x8*>(tile + ((wave * 4 + hy) * kHalo + (m + hx)) * kPixStride + kb * 8);
+#pragma unroll
+            for (int mt = 0; mt < 4; mt++) {
+                const int ky = FLIP ? 2 - (hy - mt) : hy - mt;
+                if (ky < 0 || ky > 2) continue;
+                acc[mt][0] = mfma16(B[ky * 3 + kx][0], A, acc[mt][0]);
+                acc[mt][1] = mfma16(B[ky * 3 + kx][1], A, acc[mt][1]);
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ void loadFragments(const bf16x8* __restrict__ wsw, int lane, bf16x8 (&B)[9][2]) {
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+        B[t][0] = wsw[(t * 2 + 0) * 64 + lane];
+        B[t][1] = wsw[(t * 2 + 1) * 64 + lane];
     }
 }
 
@@ -53,56 +141,39 @@ __device__ __forceinline__ void stageHalo(__bf16* tile, const __bf16* __restrict
 //   EPI_RELU_BF16   out = bf16(max(conv + bias, 0))                      hidden layers
 //   EPI_LINEAR_F32  out = f32(conv + bias)                               the logits layer
 //   EPI_MASK_BF16   out = bf16(conv * (mask > 0))                        backward data pass through the layer below's
-//                                                                        ReLU; flip = 1 mirrors the taps and the
-//                                                                        fragments hold the transposed weights
+//                                                                        ReLU: mirrored taps, and the fragments hold
+//                                                                        the transposed weights
 // wsw: 9 taps x 2 N tiles x 64 lanes of bf16x8 fragments.
+// Bound by memory: 128 B per pixel and layer, 1.4 times that with the halo. One hidden layer at 1920x1080: 99 us with
+// each halo staged in turn and tiles dealt out in order, 85 us with each operand read once (convTaps), 69 us with the
+// next halo prefetched and neighbouring tiles on one XCD (3.9 TB/s of compulsory bytes, 556 TFLOP/s).
 template <int EPI>
 __global__ __launch_bounds__(256) void k_conv3x3(const __bf16* __restrict__ in, const bf16x8* __restrict__ wsw,
                                                  const float* __restrict__ bias, const __bf16* __restrict__ mask,
-                                                 void* __restrict__ out, int N, int H, int W, int flip) {
+                                                 void* __restrict__ out, int N, int H, int W) {
     __shared__ __attribute__((aligned(16))) __bf16 tile[kHalo * kHalo * kPixStride];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, kb = lane >> 4;
     bf16x8 B[9][2];
-#pragma unroll
-    for (int t = 0; t < 9; t++) {
-        B[t][0] = wsw[(t * 2 + 0) * 64 + lane];
-        B[t][1] = wsw[(t * 2 + 1) * 64 + lane];
-    }
-    // The MFMA takes the weights as its A operand and the pixels as B, so the 16x16 result is channels x pixels:
-    // lane (m, kb) holds output channels nt * 16 + kb * 4 + 0..3 of pixel m of the tile row, four consecutive
-    // channels that leave in one 8-byte (bf16) or 16-byte (f32) store.
+    loadFragments(wsw, lane, B);
     float bco[2][4] = {};
     if (EPI != EPI_MASK_BF16)
 #pragma unroll
         for (int nt = 0; nt < 2; nt++)
 #pragma unroll
             for (int i = 0; i < 4; i++) bco[nt][i] = bias[nt * 16 + kb * 4 + i];
-    const int tilesX = (W + kTile - 1) / kTile, tilesY = (H + kTile - 1) / kTile;
-    const int numTiles = N * tilesX * tilesY;
-    for (int ti = blockIdx.x; ti < numTiles; ti += gridDim.x) {
-        const int n = ti / (tilesX * tilesY);
-        const int r = ti - n * tilesX * tilesY;
-        const int y0 = (r / tilesX) * kTile, x0 = (r % tilesX) * kTile;
+    TileWalk walk(N, H, W);
+    Halo halo;
+    if (walk.valid()) halo.load(in, walk.n, H, W, walk.y0, walk.x0);
+    while (walk.valid()) {
+        const int n = walk.n, y0 = walk.y0, x0 = walk.x0;
         __syncthreads();  // the previous tile's LDS reads are done
-        stageHalo(tile, in, n, H, W, y0, x0);
+        halo.store(tile);
         __syncthreads();
+        walk.next();
+        if (walk.valid()) halo.load(in, walk.n, H, W, walk.y0, walk.x0);
         f32x4 acc[4][2];
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++) acc[mt][0] = acc[mt][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const int ky = t / 3, kx = t % 3;
-            const int hy = flip ? 2 - ky : ky, hx = flip ? 2 - kx : kx;
-#pragma unroll
-            for (int mt = 0; mt < 4; mt++) {
-                const int row = wave * 4 + mt;
-                const bf16x8 A =
-                    *reinterpret_cast<const bf16x8*>(tile + ((row + hy) * kHalo + (m + hx)) * kPixStride + kb * 8);
-                acc[mt][0] = mfma16(B[t][0], A, acc[mt][0]);
-                acc[mt][1] = mfma16(B[t][1], A, acc[mt][1]);
-            }
-        }
+        convTaps<EPI == EPI_MASK_BF16>(tile, B, wave, m, kb, acc);
         const int x = x0 + m;
 #pragma unroll
         for (int mt = 0; mt < 4; mt++) {
@@ -427,18 +498,18 @@ __global__ void k_zeroF32(float* p, size_t n) {
 static unsigned blocksFor(size_t n, int per = 256) { return unsigned((n + per - 1) / per); }
 
 hipError_t launchKpnConv(int epilogue, const void* in, const void* wsw, const float* bias, const void* mask, void* out,
-                         int N, int H, int W, int flip, int blocks, hipStream_t stream) {
+                         int N, int H, int W, int blocks, hipStream_t stream) {
     const int tiles = N * ((H + kTile - 1) / kTile) * ((W + kTile - 1) / kTile);
     const dim3 grid(unsigned(tiles < blocks ? tiles : blocks)), block(256);
     const __bf16* i = reinterpret_cast<const __bf16*>(in);
     const bf16x8* w = reinterpret_cast<const bf16x8*>(wsw);
     const __bf16* mk = reinterpret_cast<const __bf16*>(mask);
     if (epilogue == EPI_RELU_BF16)
-        hipLaunchKernelGGL(k_conv3x3<EPI_RELU_BF16>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W, flip);
+        hipLaunchKernelGGL(k_conv3x3<EPI_RELU_BF16>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W);
     else if (epilogue == EPI_LINEAR_F32)
-        hipLaunchKernelGGL(k_conv3x3<EPI_LINEAR_F32>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W, flip);
+        hipLaunchKernelGGL(k_conv3x3<EPI_LINEAR_F32>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W);
     else
-        hipLaunchKernelGGL(k_conv3x3<EPI_MASK_BF16>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W, flip);
+        hipLaunchKernelGGL(k_conv3x3<EPI_MASK_BF16>, grid, block, 0, stream, i, w, bias, mk, out, N, H, W);
     return hipGetLastError();
 }
 
