@@ -30,13 +30,13 @@ constexpr int kConvBlocksPerCU = 2;
 
 struct KpnModel {
     DevBuf params, grads, m1, m2, wFwd, wBwd, loss;
-    DevBuf act, logits, dzA, dzB, pred, gradWork;
+    DevBuf act, logits, dzA, dzB, last, gradWork;
     size_t capPixels = 0;
     int step = 0;
     bool ready = false;
     int cuCount = 256;
     ~KpnModel() {
-        for (DevBuf* b : {&params, &grads, &m1, &m2, &wFwd, &wBwd, &loss, &act, &logits, &dzA, &dzB, &pred, &gradWork})
+        for (DevBuf* b : {&params, &grads, &m1, &m2, &wFwd, &wBwd, &loss, &act, &logits, &dzA, &dzB, &last, &gradWork})
             b->release();
     }
 };
@@ -64,6 +64,10 @@ int createModel() {
     HIP_TRY(k.wFwd.ensure(kFragBytes));
     HIP_TRY(k.wBwd.ensure(kFragBytes));
     HIP_TRY(k.loss.ensure(64));
+    if (!k.last.ptr) {
+        HIP_TRY(k.last.ensure(kKpnLastForwardBytes));
+        HIP_TRY(hipMemset(k.last.ptr, 0, kKpnLastForwardBytes));  // no forward pass yet: an empty batch
+    }
     return CRVPT_OK;
 }
 
@@ -86,11 +90,11 @@ int ensureActivations(size_t P) {
     KpnModel& k = *g_kpn;
     if (P <= k.capPixels) return CRVPT_OK;
     const size_t bf = P * kKpnChannels * 2;
+    k.capPixels = 0;  // a failed allocation leaves no pass or logits to run on the released buffers
     HIP_TRY(k.act.ensure(bf * kKpnLayers));  // inputs of the six layers
     HIP_TRY(k.logits.ensure(P * kKpnChannels * sizeof(float)));
     HIP_TRY(k.dzA.ensure(bf));
     HIP_TRY(k.dzB.ensure(bf));
-    HIP_TRY(k.pred.ensure(P * 3 * sizeof(float)));
     k.capPixels = P;
     return CRVPT_OK;
 }
@@ -111,18 +115,21 @@ int checkShape(const void* a, const void* b, int n, int h, int w) {
     return CRVPT_OK;
 }
 
-// Forward pass: features -> act[0..5] -> logits.
-int forward(const float* features, int n, int h, int w, hipStream_t s) {
+// Forward pass: features -> act[0..5] (act[0]: the packed features) -> logits (in the head's LDS) -> pred; with a target
+// also the loss and the logits' gradient dzA.
+int forward(const float* features, const float* noisy, const float* target, float* pred, int n, int h, int w,
+            hipStream_t s) {
     KpnModel& k = *g_kpn;
     const size_t P = size_t(n) * h * w;
     if (int rc = ensureActivations(P)) return rc;
-    const int blocks = k.cuCount * kConvBlocksPerCU;
-    HIP_TRY(launchKpnPack(features, actOf(k, 0, P), n, h, w, s));
-    for (int l = 0; l < kKpnLayers - 1; l++)
-        HIP_TRY(launchKpnConv(0, actOf(k, l, P), fragOf(k.wFwd, l), biasOf(k, l), nullptr, actOf(k, l + 1, P), n, h,
-                              w, blocks, s));
-    HIP_TRY(launchKpnConv(1, actOf(k, kKpnLayers - 1, P), fragOf(k.wFwd, kKpnLayers - 1),
-                          biasOf(k, kKpnLayers - 1), nullptr, k.logits.ptr, n, h, w, blocks, s));
+    const int blocks = k.cuCount * kConvBlocksPerCU, last = kKpnLayers - 1;
+    float* loss = target ? k.loss.as<float>() : nullptr;
+    HIP_TRY(launchKpnPack(features, actOf(k, 0, P), loss, n, h, w, s));
+    for (int l = 0; l < last; l++)
+        HIP_TRY(launchKpnConv(l == 0, actOf(k, l, P), fragOf(k.wFwd, l), biasOf(k, l), actOf(k, l + 1, P), n, h, w, blocks,
+                              s));
+    HIP_TRY(launchKpnConvHead(actOf(k, last, P), fragOf(k.wFwd, last), biasOf(k, last), noisy, target, pred,
+                              k.dzA.ptr, loss, k.last.ptr, n, h, w, blocks, s));
     return CRVPT_OK;
 }
 
@@ -191,27 +198,23 @@ int crvpt_kpn_compute_gradients(const float* features, const float* noisy, const
     KpnModel& k = *g_kpn;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const size_t P = size_t(n) * h * w;
-    if (int rc = forward(features, n, h, w, s)) return rc;
-    HIP_TRY(launchKpnZero(k.grads.as<float>(), kKpnParams, s));
-    HIP_TRY(launchKpnZero(k.loss.as<float>(), 1, s));
-    HIP_TRY(launchKpnHead(k.logits.as<float>(), noisy, target, k.pred.as<float>(), k.dzA.ptr, k.loss.as<float>(), n,
-                          h, w, s));
+    if (int rc = forward(features, noisy, target, nullptr, n, h, w, s)) return rc;
     const int blocks = k.cuCount * 2;  // gradient workgroups: one row of partial sums each
     HIP_TRY(k.gradWork.ensure(kpnGradWorkFloats(blocks) * sizeof(float)));
+    float* work = k.gradWork.as<float>();
     void* dz = k.dzA.ptr;
     void* dzNext = k.dzB.ptr;
-    float* gw = k.grads.as<float>();
-    float* gb = gw + size_t(kKpnLayers) * kKpnLayerParams;
     for (int l = kKpnLayers - 1; l >= 0; l--) {
-        HIP_TRY(launchKpnWeightGrad(actOf(k, l, P), dz, gw + size_t(l) * kKpnLayerParams, gb + size_t(l) * kKpnChannels,
-                                    n, h, w, blocks, k.gradWork.as<float>(), s));
+        HIP_TRY(launchKpnWeightGrad(l, actOf(k, l, P), dz, n, h, w, blocks, work, s));
         if (l > 0) {
             // gradient of the layer's input, through the ReLU that produced it
-            HIP_TRY(launchKpnConv(2, dz, fragOf(k.wBwd, l), nullptr, actOf(k, l, P), dzNext, n, h, w,
-                                  k.cuCount * kConvBlocksPerCU, s));
+            HIP_TRY(launchKpnConvBackward(dz, fragOf(k.wBwd, l), actOf(k, l, P), dzNext, n, h, w,
+                                          k.cuCount * kConvBlocksPerCU, s));
             std::swap(dz, dzNext);
         }
     }
+    float* gw = k.grads.as<float>();
+    HIP_TRY(launchKpnGradReduce(work, n, h, w, blocks, gw, gw + size_t(kKpnLayers) * kKpnLayerParams, s));
     if (loss) {
         HIP_TRY(hipMemcpyAsync(loss, k.loss.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
@@ -243,11 +246,7 @@ int crvpt_kpn_denoise(const float* features, const float* noisy, float* out, int
     if (int rc = requireModel()) return rc;
     if (int rc = checkShape(features, noisy, n, h, w)) return rc;
     if (!out) return fail(CRVPT_ERR_INVALID_ARGUMENT, "kpn_denoise: null output");
-    KpnModel& k = *g_kpn;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (int rc = forward(features, n, h, w, s)) return rc;
-    HIP_TRY(launchKpnHead(k.logits.as<float>(), noisy, nullptr, out, nullptr, nullptr, n, h, w, s));
-    return CRVPT_OK;
+    return forward(features, noisy, nullptr, out, n, h, w, reinterpret_cast<hipStream_t>(stream));
 }
 
 int crvpt_kpn_get_logits(float* out, int n, int h, int w, void* stream) {
@@ -255,8 +254,10 @@ int crvpt_kpn_get_logits(float* out, int n, int h, int w, void* stream) {
     KpnModel& k = *g_kpn;
     const size_t P = size_t(n) * h * w;
     if (!out || P == 0 || P > k.capPixels) return fail(CRVPT_ERR_INVALID_ARGUMENT, "kpn_get_logits: bad shape");
-    HIP_TRY(hipMemcpyAsync(out, k.logits.ptr, P * kKpnChannels * sizeof(float), hipMemcpyDeviceToDevice,
-                           reinterpret_cast<hipStream_t>(stream)));
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    // the forward pass keeps its logits in LDS: its last layer runs again, on the input and weights it had
+    HIP_TRY(launchKpnLogits(k.act.ptr, k.last.ptr, k.logits.as<float>(), k.cuCount * kConvBlocksPerCU, s));
+    HIP_TRY(hipMemcpyAsync(out, k.logits.ptr, P * kKpnChannels * sizeof(float), hipMemcpyDeviceToDevice, s));
     return CRVPT_OK;
 }
 

@@ -44,6 +44,7 @@ struct BatchLaunch {
 // Kernel-prediction denoiser network (kpn_net.hip): six 3x3 convolutions over 32-channel NHWC bf16 activations.
 constexpr int kKpnChannels = 32;                       // activation channels (inputs and logits zero-padded)
 constexpr int kKpnInputs = 15;                         // input feature channels
+constexpr int kKpnPacked = 16;                         // channels per pixel of the packed input features
 constexpr int kKpnTaps = 25;                           // 5x5 per-pixel filter taps (output logits)
 constexpr int kKpnLayers = 6;
 constexpr int kKpnLayerParams = kKpnChannels * kKpnChannels * 9;  // weights per layer [co][ci][ky * 3 + kx]
@@ -77,16 +78,28 @@ hipError_t launchBatch(int mode, const BatchRequest* reqs, const uint64_t* unitB
                        const uint32_t* frameOffset, float4* records, uint32_t* counter, hipStream_t stream);
 hipError_t launchSetU32(uint32_t* p, uint32_t v, hipStream_t stream);
 
-// KPN network kernels (kpn_net.hip). epilogue: 0 bias + ReLU -> bf16, 1 bias -> f32, 2 x (mask > 0) -> bf16.
-hipError_t launchKpnConv(int epilogue, const void* in, const void* wsw, const float* bias, const void* mask, void* out,
-                         int N, int H, int W, int blocks, hipStream_t stream);
-// Weight and bias gradients of one layer, added to dW / db; work: kpnGradWorkFloats(blocks) floats of partial sums.
+// KPN network kernels (kpn_net.hip). blocks: persistent workgroups at most.
+// f32 feature planes -> kKpnPacked bf16 channels per pixel; loss (nullable): cleared.
+hipError_t launchKpnPack(const float* features, void* out, float* loss, int N, int H, int W, hipStream_t stream);
+// A hidden layer (first: from packed features): bias + ReLU -> bf16. The backward data pass: x (mask > 0) -> bf16.
+hipError_t launchKpnConv(bool first, const void* in, const void* wsw, const float* bias, void* out, int N, int H, int W,
+                         int blocks, hipStream_t stream);
+hipError_t launchKpnConvBackward(const void* dz, const void* wsw, const void* mask, void* out, int N, int H, int W,
+                                 int blocks, hipStream_t stream);
+// Last layer, softmax and 5x5 filter; with a target also the loss and the logits' gradient. last: record of
+// kKpnLastForwardBytes that launchKpnLogits computes the logits from.
+constexpr size_t kKpnLastForwardBytes = 32 * 1024;
+hipError_t launchKpnConvHead(const void* in, const void* wsw, const float* bias, const float* noisy,
+                             const float* target, float* pred, void* dz, float* loss, void* last, int N, int H, int W,
+                             int blocks, hipStream_t stream);
+hipError_t launchKpnLogits(const void* act, const void* last, float* out, int blocks, hipStream_t stream);
+// Partial sums of one layer's weight and bias gradients, then the gradients of all layers from them; work:
+// kpnGradWorkFloats(blocks) floats, blocks: workgroups (rows of partial sums) per layer.
 size_t kpnGradWorkFloats(int blocks);
-hipError_t launchKpnWeightGrad(const void* x, const void* dz, float* dW, float* db, int N, int H, int W, int blocks,
-                               float* work, hipStream_t stream);
-hipError_t launchKpnPack(const float* features, void* out, int N, int H, int W, hipStream_t stream);
-hipError_t launchKpnHead(const float* logits, const float* noisy, const float* target, float* pred, void* dz,
-                         float* loss, int N, int H, int W, hipStream_t stream);
+hipError_t launchKpnWeightGrad(int layer, const void* x, const void* dz, int N, int H, int W, int blocks, float* work,
+                               hipStream_t stream);
+hipError_t launchKpnGradReduce(const float* work, int N, int H, int W, int blocks, float* dW, float* db,
+                               hipStream_t stream);
 hipError_t launchKpnAdam(float* param, const float* grad, float* m1, float* m2, int n, float lr, float beta1,
                          float beta2, float eps, float bc1, float bc2, hipStream_t stream);
 hipError_t launchKpnSwizzle(const float* w, void* fwd, void* bwd, int layers, hipStream_t stream);
