@@ -1100,6 +1100,11 @@ int crvpt_kpn_inv_iter_kernel(const float* x, const float* low_res_pred, const f
     Renderer& r = *g_r;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int h = std::min(img_h, weight_h), w = std::min(img_w, weight_w);
+    if (launchInvIterFused(x, low_res_pred, low_res_x, prev, fused_weights, out, use_previous != 0, n, c, img_h, img_w,
+                           lo_h, lo_w, weight_c, weight_h, weight_w, kernel_size, s)) {
+        HIP_TRY(hipGetLastError());
+        return CRVPT_OK;
+    }
     HIP_TRY(r.dKpn.ensure((size_t(n) * c * h * w + size_t(n) * kk * weight_h * weight_w) * sizeof(float)));
     float* base = r.dKpn.as<float>();
     float* soft = base + size_t(n) * c * h * w;

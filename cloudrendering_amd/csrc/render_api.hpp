@@ -177,6 +177,11 @@ hipError_t launchInvIterBase(const float* hiX, const float* loPred, const float*
                              const float* weights, float* out, bool usePrevious, int N, int C, int imgH, int imgW,
                              int loH, int loW, int wH, int wW, int K, hipStream_t stream);
 hipError_t launchSoftmaxChannels(const float* in, float* out, int N, int Ct, int kk, int H, int W, hipStream_t stream);
+// The inverse iteration's blend, softmax and apply in one kernel, without scratch memory; false (nothing launched) where
+// the sizes have no such kernel or the output overlaps an input.
+bool launchInvIterFused(const float* hiX, const float* loPred, const float* loX, const float* prev,
+                        const float* weights, float* out, bool usePrevious, int N, int C, int imgH, int imgW, int loH,
+                        int loW, int Ct, int wH, int wW, int K, hipStream_t stream);
 // Floats of the inverse-iteration apply's static scratch array (128 MiB): the base image (N*C*h*w) and the
 // normalised weights (N*K*K*wH*wW) of one call.
 constexpr size_t kKpnNoAllocScratchFloats = size_t(32) << 20;

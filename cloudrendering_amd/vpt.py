@@ -157,7 +157,7 @@ def per_pixel_kernel_forward(image, weights, kernel_size: int):
     weights = _dev4(weights, "weights")
     n, c, h, w = (int(v) for v in image.shape)
     wh, ww = int(weights.shape[2]), int(weights.shape[3])
-    out = torch.zeros((n, c, min(h, wh), min(w, ww)), dtype=torch.float32, device=image.device)
+    out = torch.empty((n, c, min(h, wh), min(w, ww)), dtype=torch.float32, device=image.device)
     stream = torch.cuda.current_stream(image.device).cuda_stream
     call("crvpt_kpn_per_pixel_kernel", ctypes.c_void_p(image.data_ptr()), ctypes.c_void_p(weights.data_ptr()),
          ctypes.c_void_p(out.data_ptr()), n, c, h, w, wh, ww, int(kernel_size), ctypes.c_void_p(stream))
@@ -176,7 +176,7 @@ def inv_iter_kernel(x, low_res_pred, low_res_x, prev, fused_weights, kernel_size
     n, c, h, w = (int(v) for v in x.shape)
     lh, lw = int(low_res_x.shape[2]), int(low_res_x.shape[3])
     wc, wh, ww = (int(v) for v in fused_weights.shape[1:])
-    out = torch.zeros((n, c, min(h, wh), min(w, ww)), dtype=torch.float32, device=x.device)
+    out = torch.empty((n, c, min(h, wh), min(w, ww)), dtype=torch.float32, device=x.device)
     stream = torch.cuda.current_stream(x.device).cuda_stream
     call("crvpt_kpn_inv_iter_kernel", ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(low_res_pred.data_ptr()),
          ctypes.c_void_p(low_res_x.data_ptr()), ctypes.c_void_p(prev.data_ptr()),
