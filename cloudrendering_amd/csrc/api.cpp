@@ -184,7 +184,7 @@ struct Renderer {
     // ---- device state ----
     hipStream_t stream = nullptr;
     DevBuf dRaw, dNorm, dNvdb, dMajorant, dRrt, dDecomp, dEnv, dAcc, dPaths, dCounter, dStage, dRays, dParams;
-    DevBuf dSvMin, dSvMax, dSvAvg, dDen0, dDen1, dStats, dFeat, dFeatAcc, dSvgf, dKpn, dBlockLeaf, dBlockTile, dBlockBad;
+    DevBuf dSvMin, dSvMax, dSvAvg, dDen0, dDen1, dStats, dFeat, dFeatAcc, dSvgf, dKpn, dTrans, dBlockLeaf, dBlockTile, dBlockBad;
     // flat 8^3-block index of the NanoVDB grid (NanoGrid::blockLeaf), valid for volume version blockTableVersion
     bool blockTableOk = false;
     uint64_t blockTableVersion = ~0ull;
@@ -209,6 +209,7 @@ struct Renderer {
     uint32_t frameCount = 0;
     uint32_t globalFrameNumber = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evT0 = nullptr, evT1 = nullptr;
+    hipEvent_t evTrans = nullptr;  // the last use of dTrans
     double lastPathMs = 0.0, lastTotalMs = 0.0;
     uint64_t lastPaths = 0;
     int lastLaunches = 0;
@@ -811,6 +812,7 @@ int crvpt_initialize(void) {
         HIP_TRY(hipEventCreate(&r->ev1));
         HIP_TRY(hipEventCreate(&r->evT0));
         HIP_TRY(hipEventCreate(&r->evT1));
+        HIP_TRY(hipEventCreateWithFlags(&r->evTrans, hipEventDisableTiming));
         const double eye[3] = {0.0, 0.0, 0.8}, ctr[3] = {0.0, 0.0, -0.2}, up[3] = {0.0, 1.0, 0.0};
         r->view = lookAt(eye, ctr, up);
         // LightEditorWidget constructor (LightEditorWidget.cpp:51-63): one white point light, view orientation.
@@ -842,13 +844,14 @@ int crvpt_cleanup(void) {
         releaseBatch();
         for (DevBuf* b : {&r->dRaw, &r->dNorm, &r->dNvdb, &r->dMajorant, &r->dRrt, &r->dDecomp, &r->dEnv, &r->dAcc,
                           &r->dPaths, &r->dCounter, &r->dStage, &r->dRays, &r->dSvMin, &r->dSvMax, &r->dSvAvg,
-                          &r->dDen0, &r->dDen1, &r->dStats, &r->dFeat, &r->dFeatAcc, &r->dSvgf, &r->dKpn,
+                          &r->dDen0, &r->dDen1, &r->dStats, &r->dFeat, &r->dFeatAcc, &r->dSvgf, &r->dKpn, &r->dTrans,
                           &r->dBlockLeaf, &r->dBlockTile, &r->dBlockBad, &r->dParams})
             b->release();
         (void)hipEventDestroy(r->ev0);
         (void)hipEventDestroy(r->ev1);
         (void)hipEventDestroy(r->evT0);
         (void)hipEventDestroy(r->evT1);
+        (void)hipEventDestroy(r->evTrans);
         (void)hipStreamDestroy(r->stream);
         delete r;
         g_r = nullptr;
@@ -1768,8 +1771,15 @@ int crvpt_transmittance_batch(int estimator, int n_rays, const float* origins, c
         m2o = m2 ? dM2 : nullptr;
     }
     HIP_TRY(hipEventRecord(r.ev0, s));
+    // the estimates of several samples per ray share one buffer: a call on another stream waits for the last one's
+    const size_t work = transmittanceWorkBytes(n_rays, n_samples);
+    if (work > 0) {
+        HIP_TRY(r.dTrans.ensure(work));
+        HIP_TRY(hipStreamWaitEvent(s, r.evTrans, 0));
+    }
     HIP_TRY(launchTransmittance(P, sp ? nullptr : &dg, sp ? &ng : nullptr, S, estimator, o, d, tm, n_rays, n_samples,
-                                seed, mo, m2o, s));
+                                seed, mo, m2o, r.dTrans.ptr, r.cuCount, s));
+    if (work > 0) HIP_TRY(hipEventRecord(r.evTrans, s));
     HIP_TRY(hipEventRecord(r.ev1, s));
     HIP_TRY(hipEventRecord(r.evT1, s));
     if (!on_device) {

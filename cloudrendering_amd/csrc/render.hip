@@ -153,95 +153,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(poolWaves<M
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Helpers of the batched residual-ratio and decomposition transmittance queries (reference traversal order).
-// ------------------------------------------------------------------------------------------------------------
-// Per-lane work counters of the transmittance estimators (density taps, supervoxel table reads).
-struct WorkCount {
-    uint32_t taps = 0;
-    uint32_t svReads = 0;
-};
-
-CRVPT_DEV float signf(float v) { return v > 0.0f ? 1.0f : (v < 0.0f ? -1.0f : 0.0f); }
-CRVPT_DEV float fractf(float v) { return v - floorf(v); }
-
-CRVPT_DEV bool refInside(const SupervoxelGrid& S, int x, int y, int z) {
-    return x >= 0 && y >= 0 && z >= 0 && x < S.refGrid[0] && y < S.refGrid[1] && z < S.refGrid[2];
-}
-CRVPT_DEV size_t refIndex(const SupervoxelGrid& S, int x, int y, int z) {
-    return (size_t(z) * S.refGrid[1] + y) * S.refGrid[0] + x;
-}
-CRVPT_DEV V3 gridDims(const SceneParams& P) {
-    return v3(P.worldToTex[0] * (P.boxMax[0] - P.boxMin[0]), P.worldToTex[1] * (P.boxMax[1] - P.boxMin[1]),
-              P.worldToTex[2] * (P.boxMax[2] - P.boxMin[2]));
-}
-
-struct RefDda {
-    int step[3];
-    float tMax[3], tDelta[3];
-    int idx[3];
-};
-
-CRVPT_DEV bool refDdaInit(const SceneParams& P, const SupervoxelGrid& S, V3 x, V3 w, float dTotal, RefDda& q) {
-    const V3 dims = gridDims(P);
-    const V3 boxDelta = v3(P.boxMax) - v3(P.boxMin);
-    const V3 sp = (x - v3(P.boxMin)) / boxDelta * dims / v3(float(S.refSize));
-    const V3 ep = (x + w * dTotal - v3(P.boxMin)) / boxDelta * dims / v3(float(S.refSize));
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const float s0 = comp(sp, a), e0 = comp(ep, a);
-        const int st = int(signf(e0 - s0));
-        const float td = st != 0 ? fminf(float(st) / (e0 - s0), 1e7f) : 1e7f;
-        q.step[a] = st;
-        q.tDelta[a] = td;
-        q.tMax[a] = st > 0 ? td * (1.0f - fractf(s0)) : td * fractf(s0);
-        q.idx[a] = int(floorf(s0));
-    }
-    return !(q.step[0] == 0 && q.step[1] == 0 && q.step[2] == 0);
-}
-
-CRVPT_DEV void refDdaAdvance(RefDda& q) {
-    int a;
-    if (q.tMax[0] < q.tMax[1]) a = q.tMax[0] < q.tMax[2] ? 0 : 2;
-    else a = q.tMax[1] < q.tMax[2] ? 1 : 2;
-    q.idx[a] += q.step[a];
-    q.tMax[a] += q.tDelta[a];
-}
-
-CRVPT_DEV void refSvBounds(const SceneParams& P, const SupervoxelGrid& S, const int idx[3], V3& mn, V3& mx) {
-    const V3 dims = gridDims(P);
-    const V3 boxDelta = v3(P.boxMax) - v3(P.boxMin);
-    const V3 lo = v3(float(idx[0] * S.refSize), float(idx[1] * S.refSize), float(idx[2] * S.refSize));
-    const V3 hi = lo + v3(float(S.refSize));
-    mn = lo / dims * boxDelta + v3(P.boxMin);
-    mx = hi / dims * boxDelta + v3(P.boxMin);
-}
-
-template <class Grid>
-CRVPT_DEV float rrtEstimator(const SceneParams& P, const Grid& grid, Rng& rng, V3 x, V3 w, float dStart, float dEnd,
-                             float T, float& wSum, float& resT, float& resDist, float muC, float muR,
-                             WorkCount& wc, typename Grid::Cache& gc) {
-    const float Tc = __expf(-muC * (dEnd - dStart));
-    float Tr = 1.0f;
-    float dist = dStart;
-    while (true) {
-        const float t = rng.exponential() / muR;
-        x += w * t;
-        dist += t;
-        if (dist >= dEnd) break;
-        const float rho = density(grid, P, rng, x, gc);
-        wc.taps++;
-        Tr *= 1.0f - (P.extinction * rho - muC) / muR;
-        const float Tlocal = T * Tr * __expf(-muC * (dist - dStart));
-        wSum += Tlocal;
-        if (rng.uniform() < Tlocal / wSum) {
-            resT = Tlocal;
-            resDist = dist;
-        }
-    }
-    return Tc * Tr;
-}
-
-// ------------------------------------------------------------------------------------------------------------
 // Accumulation: running mean over all frames since the last reset (Clouds.glsl:172-179), summed per pixel in
 // sample order, then written as [C, H, W] float32 (alpha = 1) when requested.
 // ------------------------------------------------------------------------------------------------------------
@@ -447,142 +358,6 @@ __global__ void k_featureOut(int map, FeatureAcc A, const float4* __restrict__ r
 __global__ void k_zeroU32(uint32_t* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0u;
-}
-
-// ------------------------------------------------------------------------------------------------------------
-// Batched transmittance queries.
-// ------------------------------------------------------------------------------------------------------------
-template <class Grid>
-CRVPT_DEV float transmittanceWalker(const SceneParams& P, const SupervoxelGrid& S, const Grid& grid, Rng& rng, V3 o,
-                                    V3 d, float limit, bool binary) {
-    Walker W;
-    if (!walkerStart<VPT_DELTA_TRACKING>(W, P, S, o, d, limit)) return 1.0f;
-    typename Grid::Cache gc;
-    float T = 1.0f;
-    while (true) {
-        const int ev = walkStep(W, rng, P, S);
-        if (ev == WALK_END) break;
-        if (ev != WALK_COLLIDE) continue;
-        const float rho = density(grid, P, rng, W.o + W.w * W.t, gc);
-        const float pReal = P.extinction * rho / W.mu;
-        if (binary) {
-            if (rng.uniform() < pReal) return 0.0f;
-        } else {
-            T *= 1.0f - pReal;
-        }
-    }
-    return T;
-}
-
-template <class Grid>
-CRVPT_DEV float transmittanceRrt(const SceneParams& P, const SupervoxelGrid& S, const Grid& grid, Rng& rng, V3 x,
-                                 V3 w, float limit) {
-    const V3 eps = v3(1e-6f);
-    float tMinVal, tMaxVal;
-    if (!rayBoxIntersect(v3(P.boxMin) + eps, v3(P.boxMax) - eps, x, w, tMinVal, tMaxVal)) return 1.0f;
-    x += w * tMinVal;
-    const V3 oldX = x;
-    const float lim = limit - tMinVal;
-    RefDda q;
-    if (!refDdaInit(P, S, x, w, tMaxVal - tMinVal, q)) return 1.0f;
-    float T = 1.0f, wSum = 0.0f, resT = 0.0f, resDist = 0.0f;
-    WorkCount wc;
-    typename Grid::Cache gc;
-    while (refInside(S, q.idx[0], q.idx[1], q.idx[2])) {
-        const size_t si = refIndex(S, q.idx[0], q.idx[1], q.idx[2]);
-        const float muC = S.rrt[2 * si], muR = S.rrt[2 * si + 1];
-        V3 mn, mx;
-        refSvBounds(P, S, q.idx, mn, mx);
-        float a = 0.0f, b = 0.0f;
-        rayBoxIntersect(mn, mx, oldX, w, a, b);
-        b = fminf(b, lim);
-        if (b > a) T *= rrtEstimator(P, grid, rng, oldX + w * a, w, a, b, T, wSum, resT, resDist, muC, muR, wc, gc);
-        refDdaAdvance(q);
-    }
-    return T;
-}
-
-template <class Grid>
-CRVPT_DEV float transmittanceDecomposition(const SceneParams& P, const SupervoxelGrid& S, const Grid& grid, Rng& rng,
-                                           V3 x, V3 w, float limit) {
-    const V3 eps = v3(1e-6f);
-    float tMinVal, tMaxVal;
-    if (!rayBoxIntersect(v3(P.boxMin) + eps, v3(P.boxMax) - eps, x, w, tMinVal, tMaxVal)) return 1.0f;
-    const V3 dims = gridDims(P);
-    const V3 boxDelta = v3(P.boxMax) - v3(P.boxMin);
-    const V3 svSize = v3(float(S.refSize)) * boxDelta / dims;
-    x += w * tMinVal;
-    float travelled = tMinVal;
-    typename Grid::Cache gc;
-    const V3 sp = (x - v3(P.boxMin)) / boxDelta * dims / v3(float(S.refSize));
-    int ix = int(floorf(sp.x)), iy = int(floorf(sp.y)), iz = int(floorf(sp.z));
-    while (refInside(S, ix, iy, iz)) {
-        const V3 minP = v3(P.boxMin) + v3(float(ix), float(iy), float(iz)) * svSize;
-        const V3 maxP = minP + svSize;
-        float a = 0.0f, b = 0.0f;
-        rayBoxIntersect(minP, maxP, x, w, a, b);
-        const float dMax = b - a;
-        x += w * a;
-        travelled += a;
-        const float remaining = limit - travelled;
-        if (remaining <= 0.0f) break;
-        const float dUse = fminf(dMax, remaining);
-        const size_t si = refIndex(S, ix, iy, iz);
-        const float mmMin = S.decomp[2 * si], mmMax = S.decomp[2 * si + 1];
-        if (mmMax >= 1e-5f) {
-            const float muC = fmaxf(0.0000000001f, P.extinction * mmMin);
-            const float muR = fmaxf(0.0000000001f, P.extinction * mmMax - muC);
-            const float tc = rng.exponential() / muC;
-            float tr = 0.0f;
-            while (true) {
-                tr += rng.exponential() / muR;
-                if (tc >= dUse && tr >= dUse) break;
-                if (tc <= tr) return 0.0f;
-                const float rho = density(grid, P, rng, x + w * tr, gc);
-                if (rng.uniform() * muR < P.extinction * rho - muC) return 0.0f;
-            }
-        }
-        if (dUse < dMax) break;
-        x = x + w * dMax;
-        travelled += dMax;
-        const V3 cc = (minP + maxP) * 0.5f;
-        V3 mov = x + w * 0.00001f - cc;
-        const V3 sm = v3(signf(mov.x), signf(mov.y), signf(mov.z));
-        mov = mov * sm;
-        ix += ((mov.x >= mov.y && mov.x >= mov.z) ? 1 : 0) * int(sm.x);
-        iy += ((mov.y >= mov.x && mov.y >= mov.z) ? 1 : 0) * int(sm.y);
-        iz += ((mov.z >= mov.x && mov.z >= mov.y) ? 1 : 0) * int(sm.z);
-    }
-    return 1.0f;
-}
-
-template <class Grid>
-__global__ __launch_bounds__(256) void k_transmittance(SceneParams P, Grid grid, SupervoxelGrid S, int estimator,
-                                                       const float* __restrict__ o, const float* __restrict__ d,
-                                                       const float* __restrict__ tmax, int nRays, int nSamples,
-                                                       uint32_t seed, float* __restrict__ mean,
-                                                       float* __restrict__ m2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nRays) return;
-    const V3 x = v3(o[3 * i], o[3 * i + 1], o[3 * i + 2]);
-    const V3 w = v3(d[3 * i], d[3 * i + 1], d[3 * i + 2]);
-    const float lim = tmax ? tmax[i] : kInf;
-    double s1 = 0.0, s2 = 0.0;
-    for (int s = 0; s < nSamples; s++) {
-        Rng rng;
-        rng.init(uint32_t(i), uint32_t(s), seed ^ 0x5bd1e995u);
-        float T;
-        switch (estimator) {
-            case T_RATIO: T = transmittanceWalker(P, S, grid, rng, x, w, lim, false); break;
-            case T_RESIDUAL_RATIO: T = transmittanceRrt(P, S, grid, rng, x, w, lim); break;
-            case T_DECOMPOSITION: T = transmittanceDecomposition(P, S, grid, rng, x, w, lim); break;
-            default: T = transmittanceWalker(P, S, grid, rng, x, w, lim, true); break;
-        }
-        s1 += T;
-        s2 += double(T) * T;
-    }
-    mean[i] = float(s1 / nSamples);
-    if (m2) m2[i] = float(s2 / nSamples);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -899,21 +674,6 @@ hipError_t launchFeatureOut(int map, const FeatureAcc& acc, const float4* result
 
 hipError_t launchWriteCHW(const float4* img, uint32_t npix, float* outCHW, int channels, hipStream_t stream) {
     hipLaunchKernelGGL(k_writeCHW, dim3((npix + 255) / 256), dim3(256), 0, stream, img, npix, outCHW, channels);
-    return hipGetLastError();
-}
-
-hipError_t launchTransmittance(const SceneParams& P, const DenseGrid* dense, const NanoGrid* nano,
-                               const SupervoxelGrid& S, int estimator, const float* o, const float* d,
-                               const float* tmax, int nRays, int nSamples, uint32_t seed, float* mean, float* m2,
-                               hipStream_t stream) {
-    const dim3 grid((nRays + 255) / 256), block(256);
-    if (nano) {
-        hipLaunchKernelGGL(k_transmittance<NanoAccess>, grid, block, 0, stream, P, NanoAccess{*nano}, S, estimator,
-                           o, d, tmax, nRays, nSamples, seed, mean, m2);
-    } else {
-        hipLaunchKernelGGL(k_transmittance<DenseAccess>, grid, block, 0, stream, P, DenseAccess{*dense}, S,
-                           estimator, o, d, tmax, nRays, nSamples, seed, mean, m2);
-    }
     return hipGetLastError();
 }
 
