@@ -18,7 +18,8 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.environ.get("CRVPT_BUILD_DIR", os.path.join(PKG_DIR, "_build"))
 LIB_PATH = os.environ.get("CRVPT_LIBRARY", os.path.join(PKG_DIR, "libcrvpt.so"))
 
-HIP_SOURCES = ["render.hip", "transmittance.hip", "batch.hip", "denoise.hip", "kpn.hip", "kpn_net.hip"]
+HIP_SOURCES = ["pool_dense.hip", "pool_dense_point.hip", "pool_nano.hip", "pool_nano_point.hip", "pool_nano_wide.hip",
+               "render.hip", "transmittance.hip", "batch.hip", "denoise.hip", "kpn.hip", "kpn_net.hip"]
 CXX_SOURCES = ["api.cpp", "nanovdb_build.cpp", "kpn_model.cpp"]
 
 ARCH = os.environ.get("CRVPT_OFFLOAD_ARCH", "gfx950")
@@ -51,7 +52,7 @@ def _compile(src: str) -> str:
 
 def build(verbose: bool = True) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=8) as ex:
         objs = list(ex.map(_compile, HIP_SOURCES + CXX_SOURCES))
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc(), "-shared", f"--offload-arch={ARCH}", "-o", tmp, *objs]

@@ -1,156 +1,14 @@
-// gfx950 kernels of the volumetric path tracer.
-//
-// Work decomposition: a "unit" is one camera path (pixel p, sample s) with record slot s * (W*H) + p. Claims walk
-// the image in 16 x 16 screen tiles, all of a launch's samples of one tile before the next, so a wave's 64
-// consecutive claims are 64 neighbouring pixels of one sample (coherent primary rays) and the paths in flight read a
-// small region of the volume. A persistent grid of waves drains a global claim counter: whenever lanes of a wave have no live path, one lane claims as many units as the
-// wave has free lanes (ballot + popcount + one atomic) and the free lanes take them in lane order (mbcnt), so
-// lanes refill at any step instead of idling until the longest path of the wave ends. Each path writes its
-// radiance to its own slot; a separate kernel sums the slots of a pixel in sample order, so images are
-// bit-reproducible whatever the lane/wave schedule was.
-//
-// Free-flight sampling walks a supervoxel majorant grid (piecewise-constant majorant along the ray): an Exp(1)
-// optical budget is spent supervoxel by supervoxel, empty supervoxels cost one DDA step and no density fetch, and
-// a tentative collision is accepted with probability sigma*rho / mu_local. With the grid disabled the walker
-// degenerates to the reference's global majorant (extinction.x), i.e. the reference trackers' exact free-path
-// distribution.
+// gfx950 kernels of the volumetric path tracer around the path pool (path_pool.hpp): accumulation, feature maps,
+// supervoxel tables, the block index, the fBm generator and lookup probes.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 
 #include <algorithm>
 
-#include "path_tracer.hpp"
+#include "path_pool.hpp"
 
 namespace crvpt {
-
-#ifndef CRVPT_CLAIM_TILE
-#define CRVPT_CLAIM_TILE 16
-#endif
-// Claims walk the image in square screen tiles of this edge, all of a launch's samples of one tile before the next
-// (0: sample-major over the whole image). The paths in flight then cover a few tiles instead of a quarter of the
-// image, so the volume region they read is small enough to stay in the L2 / Infinity Cache.
-constexpr uint32_t kClaimTile = CRVPT_CLAIM_TILE;
-
-CRVPT_DEV uint32_t claimCount(const SceneParams& P) {
-    if (kClaimTile == 0u) return uint32_t(P.numUnits);
-    const uint32_t tx = (uint32_t(P.width) + kClaimTile - 1u) / kClaimTile;
-    const uint32_t ty = (uint32_t(P.height) + kClaimTile - 1u) / kClaimTile;
-    return tx * ty * kClaimTile * kClaimTile * P.numFrames;
-}
-
-// Claim index -> launch slot sample * W*H + pixel (the record index); false for padding claims outside the image.
-CRVPT_DEV bool claimToSlot(const SceneParams& P, uint32_t c, uint32_t& slot) {
-    if (kClaimTile == 0u) {
-        slot = c;
-        return true;
-    }
-    constexpr uint32_t tp = kClaimTile * kClaimTile;
-    const uint32_t w = uint32_t(P.width), h = uint32_t(P.height);
-    const uint32_t tx = (w + kClaimTile - 1u) / kClaimTile;
-    const uint32_t perTile = tp * P.numFrames;
-    const uint32_t tile = udiv31(c, P.divTileClaims), rem = c - tile * perTile;
-    const uint32_t s = rem / tp, q = rem - s * tp;
-    const uint32_t ty = udiv31(tile, P.divTilesX);
-    const uint32_t x = (tile - ty * tx) * kClaimTile + q % kClaimTile, y = ty * kClaimTile + q / kClaimTile;
-    if (x >= w || y >= h) return false;
-    slot = s * (w * h) + y * w + x;
-    return true;
-}
-
-#ifndef CRVPT_CLAIM_PARTS
-#define CRVPT_CLAIM_PARTS 32
-#endif
-// Claim partitions: the tiles are split into this many contiguous ranges, each with its own claim counter, and a
-// workgroup first drains range blockIdx.x % parts, then the following ones. Workgroups are dispatched to the 8 XCDs
-// round robin, so with a multiple of 8 ranges the paths in flight on one XCD come from a few bands of the image,
-// which keeps the volume region they read, and so the XCD's L2 working set, small; the claims also spread over many
-// counters instead of one.
-constexpr uint32_t kClaimParts = CRVPT_CLAIM_PARTS;
-#ifndef CRVPT_COUNTER_STRIDE
-#define CRVPT_COUNTER_STRIDE 32
-#endif
-// Distance in 32-bit words between the claim counters of consecutive ranges (32: one 128-byte line each).
-constexpr uint32_t kCounterStride = CRVPT_COUNTER_STRIDE;
-
-CRVPT_DEV uint32_t partBegin(const SceneParams& P, uint32_t part) {
-    if (kClaimParts == 1u) return part == 0u ? 0u : claimCount(P);
-    const uint32_t tx = (uint32_t(P.width) + kClaimTile - 1u) / kClaimTile;
-    const uint32_t ty = (uint32_t(P.height) + kClaimTile - 1u) / kClaimTile;
-    const uint32_t tiles = tx * ty;
-    return uint32_t(uint64_t(tiles) * part / kClaimParts) * (kClaimTile * kClaimTile * P.numFrames);
-}
-
-// STATS: instrumented variant that keeps the per-lane work counters and adds them to `stats` at exit; in the timed
-// variant the counters are dead code and take no registers.
-template <int MODE, class Grid, bool STATS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(poolWaves<MODE>()))) void k_pathPool(
-        SceneParams P, Grid grid, SupervoxelGrid S, float4* __restrict__ out, uint32_t* __restrict__ counter,
-        int stepsPerRefill, unsigned long long* __restrict__ stats, float4* __restrict__ feat) {
-    const int lane = __lane_id();
-    PathState st;
-    st.flags = 0;
-    st.unit = 0;
-    st.taps = 0;
-    bool exhausted = false;
-    uint32_t paths = 0;
-    Walker W;
-    W.svReads = 0;
-    typename Grid::Cache gc;
-    uint32_t part = kClaimParts == 1u ? 0u : blockIdx.x % kClaimParts;  // wave-uniform
-    uint32_t partsLeft = kClaimParts;
-    uint32_t begin = partBegin(P, part), count = partBegin(P, part + 1u) - begin;
-    while (true) {
-        // Refill until every lane holds a live path or the queue is drained: a claimed path whose camera ray misses
-        // the volume finishes inside startPath, and its lane claims again before the wave steps.
-        while (true) {
-            const bool needs = !(st.flags & PF_ALIVE) && !exhausted;
-            const uint64_t needMask = __ballot(needs);
-            if (needMask == 0) break;
-            const int leader = __ffsll((unsigned long long)needMask) - 1;
-            const uint32_t want = uint32_t(__popcll(needMask));
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&counter[part * kCounterStride], want);
-            base = __builtin_amdgcn_readfirstlane(__shfl(base, leader));  // wave-uniform: the range state in SGPRs
-            if (needs) {
-                const uint32_t c = base + uint32_t(__popcll(needMask & ((1ull << lane) - 1ull)));
-                if (c < count && claimToSlot(launchParams<MODE>(P), begin + c, st.unit)) {
-                    paths++;
-                    if (!startPath<MODE>(st, W, P, S, feat)) writePath(out, st);
-                }
-            }
-            if (base + want >= count) {
-                // this range is drained: the next one, until every range is
-                if (--partsLeft == 0u) {
-                    exhausted = true;
-                } else {
-                    part = part + 1u == kClaimParts ? 0u : part + 1u;
-                    begin = partBegin(P, part);
-                    count = partBegin(P, part + 1u) - begin;
-                }
-            }
-        }
-        if (__ballot((st.flags & PF_ALIVE) != 0) == 0) break;  // every lane is exhausted
-        for (int k = 0; k < stepsPerRefill; k++) {
-            if ((st.flags & (PF_ALIVE | PF_PENDING)) == PF_ALIVE) {
-                if (!stepPath<MODE, Grid>(st, W, P, S, grid, gc, feat)) {
-                    writePath(out, st);
-                    st.flags = 0;
-                }
-            }
-            const uint64_t pend = __ballot((st.flags & PF_PENDING) != 0);
-            if (pend != 0ull && (__popcll(pend) >= kResolveLanes || k == stepsPerRefill - 1)) {
-                if (st.flags & PF_PENDING) {
-                    if (!resolvePending<MODE, Grid>(st, W, P, S, grid, feat)) {
-                        writePath(out, st);
-                        st.flags = 0;
-                    }
-                }
-            }
-        }
-    }
-    if (STATS) flushCounters(stats, st.taps, W.svReads, paths, gc.descents());
-}
 
 // ------------------------------------------------------------------------------------------------------------
 // Accumulation: running mean over all frames since the last reset (Clouds.glsl:172-179), summed per pixel in
@@ -553,57 +411,6 @@ __global__ void k_nanoLookupWorld(NanoAccess grid, int n, const float* __restric
 // ------------------------------------------------------------------------------------------------------------
 // Host-side launchers
 // ------------------------------------------------------------------------------------------------------------
-template <int MODE, class Grid>
-static void launchPool(dim3 grid, dim3 block, hipStream_t stream, const SceneParams& P, const Grid& g,
-                       const SupervoxelGrid& S, float4* paths, uint32_t* counter, int steps,
-                       unsigned long long* stats, float4* feat) {
-    if (stats)
-        hipLaunchKernelGGL((k_pathPool<MODE, Grid, true>), grid, block, 0, stream, P, g, S, paths, counter, steps,
-                           stats, feat);
-    else
-        hipLaunchKernelGGL((k_pathPool<MODE, Grid, false>), grid, block, 0, stream, P, g, S, paths, counter, steps,
-                           stats, feat);
-}
-
-template <class Grid>
-static hipError_t launchRenderT(const SceneParams& P, const Grid& grid, const SupervoxelGrid& S, float4* paths,
-                                uint32_t* counter, const LaunchConfig& cfg, unsigned long long* stats, float4* feat,
-                                hipStream_t stream) {
-    hipLaunchKernelGGL(k_zeroU32, dim3((kClaimParts * kCounterStride + 255) / 256), dim3(256), 0, stream, counter,
-                       int(kClaimParts * kCounterStride));
-    const dim3 block(256);
-    const dim3 gridDim(cfg.numBlocks);
-    const int st = cfg.stepsPerRefill;
-    switch (P.mode) {
-        case VPT_RATIO_TRACKING:
-            launchPool<VPT_RATIO_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats, feat);
-            break;
-        case VPT_NEXT_EVENT_TRACKING:
-            launchPool<VPT_NEXT_EVENT_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats, feat);
-            break;
-        case VPT_SPECTRAL_DELTA_TRACKING:
-            launchPool<VPT_SPECTRAL_DELTA_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats,
-                                                    feat);
-            break;
-        case VPT_NEXT_EVENT_TRACKING_SPECTRAL:
-            launchPool<VPT_NEXT_EVENT_TRACKING_SPECTRAL>(gridDim, block, stream, P, grid, S, paths, counter, st,
-                                                         stats, feat);
-            break;
-        case VPT_DECOMPOSITION_TRACKING:
-            launchPool<VPT_DECOMPOSITION_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats,
-                                                   feat);
-            break;
-        case VPT_RESIDUAL_RATIO_TRACKING:
-            launchPool<VPT_RESIDUAL_RATIO_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats,
-                                                    feat);
-            break;
-        default:
-            launchPool<VPT_DELTA_TRACKING>(gridDim, block, stream, P, grid, S, paths, counter, st, stats, feat);
-            break;
-    }
-    return hipGetLastError();
-}
-
 __global__ void k_storeParams(SceneParams* __restrict__ dst, SceneParams P) {
     // word by word from the kernel argument (the struct is a whole number of 4-byte words)
     static_assert(sizeof(SceneParams) % 4 == 0, "SceneParams is copied in 4-byte words");
@@ -626,8 +433,10 @@ uint32_t maxFramesPerLaunch(int width, int height) {
 }
 
 hipError_t launchRender(const SceneParams& Pin, const DenseGrid* dense, const NanoGrid* nano, const SupervoxelGrid& S,
-                        float4* paths, uint32_t* counter, const LaunchConfig& cfg, unsigned long long* stats,
+                        float4* paths, uint32_t* counter, const LaunchConfig& cfgIn, unsigned long long* stats,
                         float4* feat, hipStream_t stream) {
+    LaunchConfig cfg = cfgIn;
+    cfg.drain.count = counter + kDrainCount;
     if (Pin.numFrames == 0u || Pin.numFrames > maxFramesPerLaunch(Pin.width, Pin.height) || !Pin.mem)
         return hipErrorInvalidValue;
     SceneParams P = Pin;
@@ -636,18 +445,19 @@ hipError_t launchRender(const SceneParams& Pin, const DenseGrid* dense, const Na
     P.divTilesX = makeDiv31(kClaimTile == 0u ? 1u : (uint32_t(P.width) + kClaimTile - 1u) / kClaimTile);
     // this launch's constants, with its frame range and claim divisors, in the device copy the kernels read
     if (const hipError_t e = launchStoreParams(const_cast<SceneParams*>(Pin.mem), P, stream)) return e;
+    hipLaunchKernelGGL(k_zeroU32, dim3((kClaimWords + 255) / 256), dim3(256), 0, stream, counter, int(kClaimWords));
     // variants: 64-bit offsets and the full index map only for NanoVDB grids of 4 GiB and more or with rotated
     // voxels, 64-bit voxel indices only for dense grids of 2^32 voxels and more; the trilinear code only for the
     // trilinear filter
     const bool tri = P.interpolation == INTERP_TRILINEAR;
     if (nano && (nano->wide || !nano->tapDiag))
-        return launchRenderT(P, NanoAccess{*nano}, S, paths, counter, cfg, stats, feat, stream);
-    if (nano && tri) return launchRenderT(P, NanoAccessNarrow{*nano}, S, paths, counter, cfg, stats, feat, stream);
-    if (nano) return launchRenderT(P, NanoAccessNarrowPoint{*nano}, S, paths, counter, cfg, stats, feat, stream);
+        return launchPoolT(P, NanoAccess{*nano}, S, paths, counter, cfg, stats, feat, stream);
+    if (nano && tri) return launchPoolT(P, NanoAccessNarrow{*nano}, S, paths, counter, cfg, stats, feat, stream);
+    if (nano) return launchPoolT(P, NanoAccessNarrowPoint{*nano}, S, paths, counter, cfg, stats, feat, stream);
     const bool small =
             uint64_t(dense->dim[0]) * uint64_t(dense->dim[1]) * uint64_t(dense->dim[2]) < (uint64_t(1) << 32);
-    if (!tri && small) return launchRenderT(P, DenseAccessPoint{*dense}, S, paths, counter, cfg, stats, feat, stream);
-    return launchRenderT(P, DenseAccess{*dense}, S, paths, counter, cfg, stats, feat, stream);
+    if (!tri && small) return launchPoolT(P, DenseAccessPoint{*dense}, S, paths, counter, cfg, stats, feat, stream);
+    return launchPoolT(P, DenseAccess{*dense}, S, paths, counter, cfg, stats, feat, stream);
 }
 
 hipError_t launchAccumulate(const float4* paths, uint32_t npix, uint32_t frames, float4* acc, uint32_t prevFrames,
@@ -761,23 +571,9 @@ hipError_t launchNanoLookupWorld(const NanoGrid& nano, int n, const float* xyz, 
     return hipGetLastError();
 }
 
-template <class Grid>
-static const void* pathPoolKernel(int mode) {
-    switch (mode) {
-        case VPT_RATIO_TRACKING: return (const void*)k_pathPool<VPT_RATIO_TRACKING, Grid, false>;
-        case VPT_NEXT_EVENT_TRACKING: return (const void*)k_pathPool<VPT_NEXT_EVENT_TRACKING, Grid, false>;
-        case VPT_SPECTRAL_DELTA_TRACKING: return (const void*)k_pathPool<VPT_SPECTRAL_DELTA_TRACKING, Grid, false>;
-        case VPT_NEXT_EVENT_TRACKING_SPECTRAL:
-            return (const void*)k_pathPool<VPT_NEXT_EVENT_TRACKING_SPECTRAL, Grid, false>;
-        case VPT_DECOMPOSITION_TRACKING: return (const void*)k_pathPool<VPT_DECOMPOSITION_TRACKING, Grid, false>;
-        case VPT_RESIDUAL_RATIO_TRACKING: return (const void*)k_pathPool<VPT_RESIDUAL_RATIO_TRACKING, Grid, false>;
-        default: return (const void*)k_pathPool<VPT_DELTA_TRACKING, Grid, false>;
-    }
-}
-
 int occupancyBlocksPerCU(int mode, bool sparse) {
     int blocks = 0;
-    const void* k = sparse ? pathPoolKernel<NanoAccessNarrowPoint>(mode) : pathPoolKernel<DenseAccessPoint>(mode);
+    const void* k = sparse ? poolKernelT<NanoAccessNarrowPoint>(mode) : poolKernelT<DenseAccessPoint>(mode);
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, 0);
     if (e != hipSuccess || blocks <= 0) return 4;
     return blocks;

@@ -28,9 +28,18 @@ constexpr int kFeatureAccArrays = 11;
 // FeatureMapTypeVpt values (0..20), for denoisers that weight by the noise level.
 constexpr int kFeatureMapRadianceVariance = 21;
 
+// States of the paths the pool hands to its drain, kDrainWords words each (words null: no drain).
+constexpr int kDrainWords = 36;
+struct DrainQueue {
+    uint32_t* words;
+    uint32_t* count;  // states saved (set by launchRender)
+};
+
 struct LaunchConfig {
     uint32_t numBlocks;      // persistent workgroups of 256 threads
     int32_t stepsPerRefill;  // walker events per lane between two refill ballots (the compaction interval)
+    uint32_t drainBlocks;    // workgroups of the drain
+    DrainQueue drain;
 };
 
 // Launch shape of the batched queue (the autotuner's parameters).
