@@ -17,7 +17,7 @@
 
 #include <stdint.h>
 
-#include "path_tracer.hpp"
+#include "path_drain.hpp"
 
 namespace crvpt {
 
@@ -57,11 +57,12 @@ CRVPT_DEV uint32_t unitPartBegin(uint32_t totalUnits, uint32_t part) {
     return uint32_t(uint64_t(totalUnits) * part / kBatchParts);
 }
 
-template <int MODE>
+// DRAIN (units of one sample): the pool leaves its last paths to k_batchDrain.
+template <int MODE, bool DRAIN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batchPoolWaves<MODE>()))) void k_batchPool(
         const BatchRequest* __restrict__ reqs, const uint64_t* __restrict__ unitBegins, int nreq, uint32_t totalUnits,
         uint32_t samplesPerUnit, const uint32_t* __restrict__ frameOffset, float4* __restrict__ records,
-        uint32_t* __restrict__ counter, int stepsPerRefill) {
+        uint32_t* __restrict__ counter, int stepsPerRefill, DrainQueue drain) {
     const int lane = __lane_id();
     const uint32_t frameOff = *frameOffset;
     PathState st;
@@ -137,7 +138,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batchPoolWa
             }
             if (__ballot(!(st.flags & PF_ALIVE) && (left > 0u || !exhausted)) == 0ull) break;
         }
-        if (__ballot((st.flags & PF_ALIVE) != 0) == 0ull) break;  // every lane is exhausted
+        // (the ballot in a variable of its own, see k_pathPool)
+        const uint64_t alive = __ballot((st.flags & PF_ALIVE) != 0);
+        if (alive == 0ull) break;                         // every lane is exhausted
+        if (DRAIN && __ballot(exhausted) != 0ull) break;  // the drain takes the live paths
         for (int k = 0; k < stepsPerRefill; k++) {
             if ((st.flags & (PF_ALIVE | PF_PENDING)) == PF_ALIVE) {
                 const BatchRequest& R = reqs[req];
@@ -152,6 +156,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batchPoolWa
             }
         }
     }
+    if (DRAIN) {
+        const uint64_t alive = __ballot((st.flags & PF_ALIVE) != 0);
+        if (alive != 0ull) saveState<MODE>(st, W, drain, alive, lane, uint32_t(req) + 1u);
+    }
+}
+
+// Traces the paths the batch pool saved to their end; a path's request is the word behind its state.
+template <int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kDrainWaves))) void k_batchDrain(
+        const BatchRequest* __restrict__ reqs, const uint64_t* __restrict__ unitBegins,
+        const uint32_t* __restrict__ frameOffset, float4* __restrict__ records, DrainQueue drain) {
+    struct Request {
+        const BatchRequest* reqs;
+        const uint64_t* unitBegins;
+        uint32_t frameOff;
+        float4* records;
+        int req;
+        LeafCache gc;
+        CRVPT_DEV void open(PathState& st, const uint32_t* words) {
+            const int r = int(words[kDrainWords - 1]) - 1;
+            if (r != req) gc = LeafCache();  // the memo holds byte offsets into the previous request's grid
+            req = r;
+            const BatchRequest& R = reqs[req];
+            const uint32_t npix = uint32_t(R.P.width) * uint32_t(R.P.height);
+            const uint32_t local = st.unit - uint32_t(unitBegins[req]);
+            const uint32_t sample = local / npix;  // a unit is one sample
+            st.pix = local - sample * npix;
+            st.frame = R.P.frameBase + frameOff + sample;
+        }
+        CRVPT_DEV void moveFrom(int from) {
+            req = __shfl(req, from);
+            gc = LeafCache();
+        }
+        CRVPT_DEV float extinction() const { return reqs[req].P.extinction; }
+        CRVPT_DEV bool step(PathState& st, Walker& W, int lg, int sub, int base) {
+            const BatchRequest& R = reqs[req];
+            return coopStep<MODE, BatchGrid>(st, W, R.P, R.S, BatchGrid{&R}, gc, nullptr, lg, sub, base);
+        }
+        CRVPT_DEV bool resolve(PathState& st, Walker& W) {
+            const BatchRequest& R = reqs[req];
+            return resolvePending<MODE, BatchGrid>(st, W, R.P, R.S, BatchGrid{&R}, nullptr);
+        }
+        CRVPT_DEV void finish(const PathState& st) {
+            records[st.unit] = make_float4(st.color.x, st.color.y, st.color.z, 0.0f);
+        }
+    } request{reqs, unitBegins, *frameOffset, records, 0, {}};
+    drainPaths<MODE>(drain, request);
 }
 
 // Per pixel of every request: the sum of its units' records in group order, divided by spp (the single-frame
@@ -184,26 +235,27 @@ __global__ void k_setU32(uint32_t* p, uint32_t v) {
     if (threadIdx.x == 0) *p = v;
 }
 
-template <int MODE>
-static const void* batchKernel() {
-    return (const void*)k_batchPool<MODE>;
-}
-
-static const void* batchPoolKernel(int mode) {
+// Calls f with the estimator as an integral constant.
+template <class F>
+static void withMode(int mode, F&& f) {
     switch (mode) {
-        case VPT_RATIO_TRACKING: return batchKernel<VPT_RATIO_TRACKING>();
-        case VPT_NEXT_EVENT_TRACKING: return batchKernel<VPT_NEXT_EVENT_TRACKING>();
-        case VPT_SPECTRAL_DELTA_TRACKING: return batchKernel<VPT_SPECTRAL_DELTA_TRACKING>();
-        case VPT_NEXT_EVENT_TRACKING_SPECTRAL: return batchKernel<VPT_NEXT_EVENT_TRACKING_SPECTRAL>();
-        case VPT_DECOMPOSITION_TRACKING: return batchKernel<VPT_DECOMPOSITION_TRACKING>();
-        case VPT_RESIDUAL_RATIO_TRACKING: return batchKernel<VPT_RESIDUAL_RATIO_TRACKING>();
-        default: return batchKernel<VPT_DELTA_TRACKING>();
+        case VPT_RATIO_TRACKING: f(std::integral_constant<int, VPT_RATIO_TRACKING>()); break;
+        case VPT_NEXT_EVENT_TRACKING: f(std::integral_constant<int, VPT_NEXT_EVENT_TRACKING>()); break;
+        case VPT_SPECTRAL_DELTA_TRACKING: f(std::integral_constant<int, VPT_SPECTRAL_DELTA_TRACKING>()); break;
+        case VPT_NEXT_EVENT_TRACKING_SPECTRAL:
+            f(std::integral_constant<int, VPT_NEXT_EVENT_TRACKING_SPECTRAL>());
+            break;
+        case VPT_DECOMPOSITION_TRACKING: f(std::integral_constant<int, VPT_DECOMPOSITION_TRACKING>()); break;
+        case VPT_RESIDUAL_RATIO_TRACKING: f(std::integral_constant<int, VPT_RESIDUAL_RATIO_TRACKING>()); break;
+        default: f(std::integral_constant<int, VPT_DELTA_TRACKING>()); break;
     }
 }
 
 int batchOccupancyBlocksPerCU(int mode, int blockSize) {
+    const void* kernel = nullptr;
+    withMode(mode, [&](auto m) { kernel = (const void*)k_batchPool<decltype(m)::value, false>; });
     int blocks = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, batchPoolKernel(mode), blockSize, 0);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, blockSize, 0);
     if (e != hipSuccess || blocks <= 0) return 1;
     return blocks;
 }
@@ -215,15 +267,34 @@ hipError_t launchSetU32(uint32_t* p, uint32_t v, hipStream_t stream) {
 
 hipError_t launchBatch(int mode, const BatchRequest* reqs, const uint64_t* unitBegins, const uint64_t* pixBegins,
                        int nreq, uint32_t totalUnits, uint64_t totalPix, const BatchLaunch& cfg,
-                       const uint32_t* frameOffset, float4* records, uint32_t* counter, hipStream_t stream) {
+                       const uint32_t* frameOffset, float4* records, uint32_t* counter, uint32_t* drainWords,
+                       uint32_t drainBlocks, hipStream_t stream) {
     if (cfg.blockSize <= 0 || cfg.blockSize > 256 || cfg.blockSize % 64 != 0 || cfg.numBlocks == 0 ||
-        cfg.samplesPerUnit == 0 || cfg.stepsPerRefill <= 0)
+        cfg.samplesPerUnit == 0 || cfg.stepsPerRefill <= 0 || (drainWords && cfg.samplesPerUnit != 1u))
         return hipErrorInvalidValue;
     for (uint32_t p = 0; p < kBatchParts; p++) hipLaunchKernelGGL(k_setU32, dim3(1), dim3(64), 0, stream, counter + p, 0u);
-    void* args[] = {(void*)&reqs,    (void*)&unitBegins, (void*)&nreq,    (void*)&totalUnits,
-                    (void*)&cfg.samplesPerUnit, (void*)&frameOffset, (void*)&records, (void*)&counter,
-                    (void*)&cfg.stepsPerRefill};
-    hipError_t e = hipLaunchKernel(batchPoolKernel(mode), dim3(cfg.numBlocks), dim3(cfg.blockSize), args, 0, stream);
+    DrainQueue drain{drainWords, counter + kBatchParts};
+    const dim3 grid(cfg.numBlocks), block(cfg.blockSize);
+    if (drainWords) hipLaunchKernelGGL(k_setU32, dim3(1), dim3(64), 0, stream, drain.count, 0u);
+    hipError_t e = hipSuccess;
+    withMode(mode, [&](auto m) {
+        constexpr int M = decltype(m)::value;
+        if constexpr (drains<M>()) {
+            if (drainWords) {
+                hipLaunchKernelGGL((k_batchPool<M, true>), grid, block, 0, stream, reqs, unitBegins, nreq, totalUnits,
+                                   cfg.samplesPerUnit, frameOffset, records, counter, cfg.stepsPerRefill, drain);
+                e = hipGetLastError();
+                if (e != hipSuccess) return;
+                hipLaunchKernelGGL(k_batchDrain<M>, dim3(drainBlocks), dim3(256), 0, stream, reqs, unitBegins,
+                                   frameOffset, records, drain);
+                e = hipGetLastError();
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_batchPool<M, false>), grid, block, 0, stream, reqs, unitBegins, nreq, totalUnits,
+                           cfg.samplesPerUnit, frameOffset, records, counter, cfg.stepsPerRefill, drain);
+        e = hipGetLastError();
+    });
     if (e != hipSuccess) return e;
     const uint64_t blocks = (totalPix + 255) / 256;
     hipLaunchKernelGGL(k_batchResolve, dim3(unsigned(blocks)), dim3(256), 0, stream, reqs, pixBegins, nreq, totalPix,

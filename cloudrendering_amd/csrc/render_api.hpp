@@ -81,10 +81,11 @@ hipError_t launchRender(const SceneParams& P, const DenseGrid* dense, const Nano
                         float4* paths, uint32_t* counter, const LaunchConfig& cfg, unsigned long long* stats,
                         float4* feat, hipStream_t stream);
 // Batched queue (batch.hip): one persistent path-pool launch over every request, then one resolve launch that writes
-// each request's image. unitBegins / pixBegins: nreq ascending first units / first pixels (device arrays).
+// each request's image. drainWords (nullable, units of one sample only): kDrainWords per lane of the pool. unitBegins / pixBegins: nreq ascending first units / first pixels (device arrays).
 hipError_t launchBatch(int mode, const BatchRequest* reqs, const uint64_t* unitBegins, const uint64_t* pixBegins,
                        int nreq, uint32_t totalUnits, uint64_t totalPix, const BatchLaunch& cfg,
-                       const uint32_t* frameOffset, float4* records, uint32_t* counter, hipStream_t stream);
+                       const uint32_t* frameOffset, float4* records, uint32_t* counter, uint32_t* drainWords,
+                       uint32_t drainBlocks, hipStream_t stream);
 hipError_t launchSetU32(uint32_t* p, uint32_t v, hipStream_t stream);
 
 // KPN network kernels (kpn_net.hip). blocks: persistent workgroups at most.
