@@ -172,8 +172,8 @@ struct SvgfInputs {
     int width, height;
 };
 struct SvgfState {
-    float4* prevNormal;
-    float4* prevDepth;
+    float4* prevGuide;  // (normal, depth) of the previous frame
+    float4* guide;      // and of this one
     float4* colorHistory;
     float4* momentsHistory;
     float4* accumMoments;
