@@ -166,6 +166,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(poolWaves<M
     if (STATS) flushCounters(stats, st.taps, W.svReads, paths, gc.descents());
 }
 
+// Starts the camera paths of a small launch, a thread per claim, for the drain to trace from their beginning: such a
+// launch needs no pool (a 64 x 64 frame spent 90 us in it, most of that on the 32 claim counters: 400 us a pass, now
+// 300). Bound by the latency of one path's start.
+template <int MODE, class Grid>
+__global__ __launch_bounds__(256) void k_pathStart(SceneParams P, SupervoxelGrid S, float4* __restrict__ out,
+                                                   float4* __restrict__ feat, DrainQueue drain) {
+    const int lane = __lane_id();
+    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+    PathState st;
+    st.flags = 0;
+    st.unit = 0;
+    st.pendRho = 0.0f;
+    Walker W{};
+    if (c < claimCount(P) && claimToSlot(launchParams<MODE>(P), c, st.unit)) {
+        if (!startPath<MODE>(st, W, P, S, feat)) {
+            writePath(out, st);
+            st.flags = 0;
+        }
+    }
+    const uint64_t alive = __ballot((st.flags & PF_ALIVE) != 0);
+    if (alive != 0ull) saveState<MODE>(st, W, drain, alive, lane, 0u);
+}
+
 // Traces the paths the pool saved to their end.
 template <int MODE, class Grid>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kDrainWaves))) void k_pathDrain(
@@ -212,8 +235,12 @@ static void launchPool(const SceneParams& P, const Grid& g, const SupervoxelGrid
     }
     if constexpr (drains<MODE>()) {
         if (Q.words) {
-            hipLaunchKernelGGL((k_pathPool<MODE, Grid, false, true>), grid, block, 0, stream, P, g, S, paths, counter,
-                               steps, stats, feat, Q);
+            if (cfg.startBlocks > 0)
+                hipLaunchKernelGGL((k_pathStart<MODE, Grid>), dim3(cfg.startBlocks), block, 0, stream, P, S, paths, feat,
+                                   Q);
+            else
+                hipLaunchKernelGGL((k_pathPool<MODE, Grid, false, true>), grid, block, 0, stream, P, g, S, paths,
+                                   counter, steps, stats, feat, Q);
             hipLaunchKernelGGL((k_pathDrain<MODE, Grid>), dim3(cfg.drainBlocks), block, 0, stream, P, g, S, paths, feat,
                                Q);
             return;

@@ -437,6 +437,12 @@ hipError_t launchRender(const SceneParams& Pin, const DenseGrid* dense, const Na
                         float4* feat, hipStream_t stream) {
     LaunchConfig cfg = cfgIn;
     cfg.drain.count = counter + kDrainCount;
+    if (cfg.startBlocks > 0) {
+        const uint64_t tile = std::max<uint64_t>(kClaimTile, 1);
+        const uint64_t claims = (uint64_t(Pin.width) + tile - 1) / tile * ((uint64_t(Pin.height) + tile - 1) / tile) *
+                                tile * tile * Pin.numFrames;
+        cfg.startBlocks = uint32_t((claims + 255) / 256);
+    }
     if (Pin.numFrames == 0u || Pin.numFrames > maxFramesPerLaunch(Pin.width, Pin.height) || !Pin.mem)
         return hipErrorInvalidValue;
     SceneParams P = Pin;

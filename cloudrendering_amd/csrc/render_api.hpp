@@ -39,6 +39,7 @@ struct LaunchConfig {
     uint32_t numBlocks;      // persistent workgroups of 256 threads
     int32_t stepsPerRefill;  // walker events per lane between two refill ballots (the compaction interval)
     uint32_t drainBlocks;    // workgroups of the drain
+    uint32_t startBlocks;    // not 0: no pool, the paths are only started for the drain (launchRender sets the count)
     DrainQueue drain;
 };
 

@@ -53,8 +53,9 @@ def test_drain_equals_pool(vpt, mode, interpolation, volume):
     vpt.set_use_lights(mode == 5)
     vpt.set_camera_position([0.1, 0.2, 0.7])
     vpt.set_camera_target([0.0, 0.0, 0.0])
-    # one path; fewer than a wave; waves of one lane group; more paths than the drain has lanes
-    for w, h, spp in ((1, 1, 1), (7, 5, 1), (64, 48, 2), (301, 203, 7)):
+    # one path; fewer than a wave; the most paths that are started for the drain alone, and the fewest that go through
+    # the pool first (2^16 and 2^17); more paths than the drain has lanes
+    for w, h, spp in ((1, 1, 1), (7, 5, 1), (256, 256, 1), (256, 257, 1), (256, 256, 2), (256, 257, 2), (301, 203, 7)):
         _same(_render(vpt, w, h, spp, False)[0], _render(vpt, w, h, spp, True)[0])
     vpt.set_sparse_value_type(0)
 
