@@ -406,7 +406,7 @@ CRVPT_DEV bool startPathAt(PathState& st, Walker& W, const SceneParams& P, const
     V3 x, w;
     cameraRay(P, cam, st, x, w);
     if (!walkerStart<MODE>(W, P, S, x, w, kInf)) {
-        finishPath(st, skyRadiance(skyParams<MODE>(P), w), false);
+        finishPath(st, skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), w), false);
         return false;
     }
     return true;
@@ -506,7 +506,7 @@ CRVPT_DEV bool scatterEvent(PathState& st, Walker& W, const SceneParams& P, cons
         }
         const float ph = evalPhase(P, W.w, dir);
         V3 L = toLight ? lightRadiance(P, p, li) * (probFactor * ph)
-                       : skyRadiance(skyParams<MODE>(P), dir) * (probFactor * ph * (4.0f * kPi));
+                       : skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), dir) * (probFactor * ph * (4.0f * kPi));
         if (isSpectral<MODE>()) L = L * vmin(st.weights, 100000.0f);
         st.mainX = p;
         st.mainW = nw;
@@ -528,7 +528,7 @@ CRVPT_DEV bool scatterEvent(PathState& st, Walker& W, const SceneParams& P, cons
     }
     if (!walkerStart<MODE>(W, P, S, p, nw, kInf, false, MODE == VPT_DECOMPOSITION_TRACKING)) {
         const V3 c = isNee<MODE>() ? st.color
-                                   : skyRadiance(skyParams<MODE>(P), nw) *
+                                   : skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), nw) *
                                          (isSpectral<MODE>() ? vmin(st.weights, 100000.0f) : v3(st.thr));
         finishPath(st, c, true);
         return false;
@@ -549,8 +549,8 @@ CRVPT_DEV bool endEvent(PathState& st, Walker& W, const SceneParams& P, const Su
     const bool hv = (st.flags & PF_HAS_VALUE) != 0;
     V3 c;
     const V3 wts = isSpectral<MODE>() ? vmin(st.weights, 100000.0f) : v3(st.thr);
-    if (isNee<MODE>()) c = hv ? st.color : st.color + skyRadiance(skyParams<MODE>(P), W.w) * wts;
-    else c = skyRadiance(skyParams<MODE>(P), W.w) * wts;
+    if (isNee<MODE>()) c = hv ? st.color : st.color + skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), W.w) * wts;
+    else c = skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), W.w) * wts;
     finishPath(st, c, hv);
     return false;
 }
@@ -561,7 +561,7 @@ CRVPT_DEV bool endEvent(PathState& st, Walker& W, const SceneParams& P, const Su
 CRVPT_DEV bool rrtTraversalEnd(PathState& st, Walker& W, const SceneParams& P, const SupervoxelGrid& S) {
     constexpr int MODE = VPT_RESIDUAL_RATIO_TRACKING;
     const uint4 e = pathBlock(P, st, kEventSpace | st.events++);
-    st.color += skyRadiance(skyParams<MODE>(P), W.w) * st.thr;
+    st.color += skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), W.w) * st.thr;
     const uint32_t iteration = st.flags >> kBounceShift;
     if (u01(e.x) > st.wSum || iteration >= 10u) {
         finishPath(st, st.color, true);
@@ -575,7 +575,7 @@ CRVPT_DEV bool rrtTraversalEnd(PathState& st, Walker& W, const SceneParams& P, c
     st.resT = 0.0f;
     st.resDist = 0.0f;
     if (!walkerStart<MODE>(W, P, S, x, nw, kInf)) {
-        st.color += skyRadiance(skyParams<MODE>(P), nw) * st.thr;
+        st.color += skyRadiance<isNee<MODE>()>(skyParams<MODE>(P), nw) * st.thr;
         finishPath(st, st.color, true);
         return false;
     }
