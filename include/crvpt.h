@@ -282,7 +282,8 @@ int crvpt_batch_add_request(float* out, int channels, int height, int width, int
  * launch configuration are unchanged. Asynchronous: synchronise the stream before reading the outputs. */
 int crvpt_batch_render(uint32_t frame_offset, void* stream);
 /* Launch configuration {workgroups (0 = occupancy limit x CUs), threads per workgroup (64..256, multiple of 64),
- * walker steps between refills (compaction interval), samples per claimed unit (paths per lane)}. */
+ * walker steps between refills (compaction interval), samples per claimed unit (paths per lane; an upper bound, a
+ * batch with few units per lane takes fewer)}. */
 int crvpt_batch_set_launch_config(int blocks, int block_size, int steps_per_refill, int samples_per_unit);
 int crvpt_batch_get_launch_config(int32_t config[4]);
 /* Times candidate launch configurations on the batch with spp / spp_divisor samples per request (coordinate descent
