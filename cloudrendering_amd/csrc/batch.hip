@@ -25,12 +25,14 @@ namespace crvpt {
 struct BatchGrid {
     const BatchRequest* R;
     using Cache = LeafCache;
+    template <bool FUSE_YZ>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, LeafCache& c) const {
         if (R->P.sparse) return NanoAccess{R->nano}.lookupWorldJ(P, pos, jx, jy, jz, c);
-        return DenseAccess{R->dense}.lookupWorldJ(P, pos, jx, jy, jz);
+        return DenseAccess{R->dense}.lookupWorldJ<FUSE_YZ>(P, pos, jx, jy, jz);
     }
 };
 // Batches write no feature maps.
+template <bool FUSE>
 CRVPT_DEV V3 cloudFiniteDifference(const BatchGrid&, const SceneParams&, const PathState&, V3) { return v3(0.0f); }
 
 // Last request r with begins[r] <= q (begins ascending, begins[0] = 0).

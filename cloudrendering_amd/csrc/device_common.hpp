@@ -292,6 +292,12 @@ struct NoCache {
     CRVPT_DEV uint32_t descents() const { return 0u; }
 };
 
+// a + b for a product a: rounded before the sum (never fused into one FMA).
+CRVPT_DEV V3 plainAdd(V3 a, V3 b) {
+#pragma clang fp contract(off)
+    return {a.x + b.x, a.y + b.y, a.z + b.z};
+}
+
 // TRI: the trilinear filter is compiled in; the path kernels run TRI = false for the point filters (nearest,
 // stochastic), where the eight-tap code would only hold registers. The TRI = false variant also indexes voxels with
 // 32-bit arithmetic: the launcher uses it only for grids below 2^32 voxels.
@@ -322,18 +328,37 @@ struct DenseAccessT {
             const float c11 = lerpf(voxel(i, j + 1, k + 1), voxel(i + 1, j + 1, k + 1), a);
             return lerpf(lerpf(c00, c10, b), lerpf(c01, c11, b), c);
         }
-        if (P.interpolation == INTERP_STOCHASTIC) u = u + v3(jx, jy, jz);
+        if (P.interpolation == INTERP_STOCHASTIC) u = plainAdd(u, v3(jx, jy, jz));
         return voxel(int(floorf(u.x)), int(floorf(u.y)), int(floorf(u.z)));
     }
     CRVPT_DEV V3 toTex(const SceneParams& P, V3 pos) const {
         return v3((pos.x - P.boxMin[0]) * P.worldToTex[0], (pos.y - P.boxMin[1]) * P.worldToTex[1],
                   (pos.z - P.boxMin[2]) * P.worldToTex[2]);
     }
-    CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz) const {
-        return lookupTex(P, toTex(P, pos), jx, jy, jz);
+    // toTex plus a jitter in one rounding (x always, y and z with FUSE_YZ) or in two.
+    template <bool FUSE_YZ>
+    CRVPT_DEV V3 toTexJ(const SceneParams& P, V3 pos, float jx, float jy, float jz) const {
+        const V3 d = v3(pos.x - P.boxMin[0], pos.y - P.boxMin[1], pos.z - P.boxMin[2]);
+        const float x = fmaf(d.x, P.worldToTex[0], jx);
+        if (FUSE_YZ) return v3(x, fmaf(d.y, P.worldToTex[1], jy), fmaf(d.z, P.worldToTex[2], jz));
+        const V3 u = plainAdd(v3(0.0f, d.y * P.worldToTex[1], d.z * P.worldToTex[2]), v3(0.0f, jy, jz));
+        return v3(x, u.y, u.z);
     }
+    // The tap of the path trackers. FUSE_YZ (fusedTap): the rounding of the point filter's texel coordinate. It is
+    // written out because a path may be traced in several kernels (pool, start, drain), which hand it over at a time
+    // that depends on the schedule: left to the compiler, one kernel fused this sum and another did not, and about one
+    // path in 10^6 read another voxel in the drain than it would have read in the pool.
+    template <bool FUSE_YZ>
+    CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz) const {
+        if (TRI) return lookupTex(P, toTex(P, pos), jx, jy, jz);
+        // (a jitter of 0 leaves the product of the other filters as it is)
+        const bool jitter = P.interpolation == INTERP_STOCHASTIC;
+        const V3 u = toTexJ<FUSE_YZ>(P, pos, jitter ? jx : 0.0f, jitter ? jy : 0.0f, jitter ? jz : 0.0f);
+        return voxel(int(floorf(u.x)), int(floorf(u.y)), int(floorf(u.z)));
+    }
+    template <bool FUSE_YZ>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, NoCache&) const {
-        return lookupTex(P, toTex(P, pos), jx, jy, jz);
+        return lookupWorldJ<FUSE_YZ>(P, pos, jx, jy, jz);
     }
     CRVPT_DEV float lookupWorld(const SceneParams& P, Rng& rng, V3 pos) const {
         float jx = 0.0f, jy = 0.0f, jz = 0.0f;

@@ -186,6 +186,11 @@ struct NanoAccessT {
         LeafCache c;
         return lookupWorldJ(P, pos, jx, jy, jz, c);
     }
+    // The path trackers' form: the rounding choice concerns dense grids only (DenseAccessT::lookupWorldJ).
+    template <bool FUSE_YZ>
+    CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, LeafCache& cache) const {
+        return lookupWorldJ(P, pos, jx, jy, jz, cache);
+    }
     CRVPT_DEV float lookupWorld(const SceneParams& P, Rng& rng, V3 pos, LeafCache& cache) const {
         float jx = 0.0f, jy = 0.0f, jz = 0.0f;
         if (P.interpolation == INTERP_STOCHASTIC) {

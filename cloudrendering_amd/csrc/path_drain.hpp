@@ -20,7 +20,9 @@ namespace crvpt {
 // group of lanes that looks up to kDrainGroup steps ahead (coopStep): the random numbers of a step depend on its index
 // alone, and the next tentative collisions of a free path on nothing but them, so the group's lanes evaluate the steps'
 // random blocks and density taps side by side and only the decisions follow in order. Every path makes the same steps
-// with the same operations as in the pool.
+// with the same operations as in the pool, and they have to round alike: when a wave hands a path over depends on the
+// schedule. Where the compiler's own choice of fused multiply-adds differs between the kernels the operation is written
+// out (DenseAccessT::lookupWorldJ, cloudFiniteDifference); the tests compare whole images bit for bit.
 // Kernel times in ms, pool alone -> pool and drain, for 100^2 x 1, 512^2 x 1, 1024^2 x 1, x 4 and x 16 samples:
 //   dense 128^3, delta         0.86 -> 0.42   1.06 -> 0.81   1.73 -> 1.25   3.27 -> 2.60   8.84 -> 8.29
 //   dense 128^3, next-event    7.40 -> 3.23   10.6 -> 6.44   14.0 -> 9.61   22.9 -> 18.8
@@ -135,8 +137,7 @@ CRVPT_DEV bool coopStep(PathState& st, Walker& W, const SceneParams& P, const Su
     const bool control = MODE == VPT_DECOMPOSITION_TRACKING && xi * mu < muC;
     const bool collide = ev == WALK_COLLIDE;
     float rho = 0.0f;
-    if (collide && !control)
-        rho = grid.lookupWorldJ(P, W.o + W.w * t, jitterHi(r.y), jitterLo(r.y), jitterHi(r.z), gc);
+    if (collide && !control) rho = tapDensity<MODE>(grid, P, W.o + W.w * t, r, gc);
     const uint64_t group = (~0ull >> (64 - G)) << base;
     if (MODE == VPT_RESIDUAL_RATIO_TRACKING) {
         const float factor = 1.0f - (P.extinction * rho - muC) * rcpf(mu);
@@ -207,7 +208,7 @@ CRVPT_DEV bool coopStep(PathState& st, Walker& W, const SceneParams& P, const Su
     const bool absorbed = MODE != VPT_RATIO_TRACKING && xiAt < P.absorption * pRealAt;
     if (absorbed || bounceLimit) {
         if (absorbed)
-            recordFirst<MODE>(st, P, grid, feat, W.o + W.w * W.t, isNee<MODE>() ? W.w : v3(0.0f), 0.0f,
+            recordFirst<MODE, false>(st, P, grid, feat, W.o + W.w * W.t, isNee<MODE>() ? W.w : v3(0.0f), 0.0f,
                               rhoAt * (isNee<MODE>() ? P.extinctionMax : P.extinction), W.t);
         finishPath(st, isNee<MODE>() ? st.color : v3(0.0f), true);
         return false;

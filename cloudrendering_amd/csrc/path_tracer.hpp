@@ -327,6 +327,18 @@ CRVPT_DEV float uOpen(uint32_t x) { return float((x >> 8) + 1u) * (1.0f / 167772
 CRVPT_DEV float jitterHi(uint32_t x) { return (float(x >> 16) + 0.5f) * (1.0f / 65536.0f) - 0.5f; }
 CRVPT_DEV float jitterLo(uint32_t x) { return (float(x & 0xFFFFu) + 0.5f) * (1.0f / 65536.0f) - 0.5f; }
 
+// Rounding of a dense grid's point-filtered tap (DenseAccessT::toTexJ), by estimator: what the compiler made of each
+// pool kernel when the rounding was its choice, kept so that images keep their bits.
+template <int MODE>
+constexpr bool fusedTap() {
+    return MODE == VPT_RATIO_TRACKING || walksReferenceTable<MODE>();
+}
+// Density at p with the sub-voxel jitter of step block r.
+template <int MODE, class Grid>
+CRVPT_DEV float tapDensity(const Grid& grid, const SceneParams& P, V3 p, uint4 r, typename Grid::Cache& gc) {
+    return grid.template lookupWorldJ<fusedTap<MODE>()>(P, p, jitterHi(r.y), jitterLo(r.y), jitterHi(r.z), gc);
+}
+
 // A finished path leaves its radiance in st.color and whether it met the medium in PF_HAS_VALUE; the kernel that
 // runs it stores the result (one record per path, or a sum over the samples of a batch unit).
 CRVPT_DEV void finishPath(PathState& st, V3 c, bool hasValue) {
@@ -424,17 +436,21 @@ CRVPT_DEV bool startPath(PathState& st, Walker& W, const SceneParams& P, const S
 
 // getCloudFiniteDifference (VptUtils.glsl:726-748) at p for the normal feature map: central differences of the
 // normalised grid one texel apart around the (stochastically jittered) texel, scaled by 100 / dim, normalised; the
-// reference returns 0 for NanoVDB grids.
-template <bool WIDE, bool TRI>
+// reference returns 0 for NanoVDB grids. FUSE: the jittered texel coordinate in one rounding or in two, written out for
+// the same reason as the tap's (DenseAccessT::lookupWorldJ).
+template <bool FUSE, bool WIDE, bool TRI>
 CRVPT_DEV V3 cloudFiniteDifference(const NanoAccessT<WIDE, TRI>&, const SceneParams&, const PathState&, V3) {
     return v3(0.0f);
 }
-template <bool TRI>
+template <bool FUSE, bool TRI>
 CRVPT_DEV V3 cloudFiniteDifference(const DenseAccessT<TRI>& grid, const SceneParams& P, const PathState& st, V3 p) {
-    V3 u = grid.toTex(P, p);
+    V3 u;
     if (P.interpolation == INTERP_STOCHASTIC) {
         const uint4 b = pathBlock(P, st, kFeatureBlock);
-        u = u + v3(u01(b.x) - 0.5f, u01(b.y) - 0.5f, u01(b.z) - 0.5f);
+        const float jx = u01(b.x) - 0.5f, jy = u01(b.y) - 0.5f, jz = u01(b.z) - 0.5f;
+        u = FUSE ? grid.template toTexJ<true>(P, p, jx, jy, jz) : plainAdd(grid.toTex(P, p), v3(jx, jy, jz));
+    } else {
+        u = grid.toTex(P, p);
     }
     const V3 dim = v3(P.worldToTex[0] * (P.boxMax[0] - P.boxMin[0]), P.worldToTex[1] * (P.boxMax[1] - P.boxMin[1]),
                       P.worldToTex[2] * (P.boxMax[2] - P.boxMin[2]));
@@ -453,12 +469,12 @@ CRVPT_DEV V3 cloudFiniteDifference(const DenseAccessT<TRI>& grid, const ScenePar
 // First scattering or absorption event of the path (the ScatterEvent the trackers fill, Clouds.glsl:91-96): its
 // position, depth (distance along the camera ray), outgoing direction and phase pdf, extinction-scaled density and
 // the finite-difference normal, written once per path for the feature maps.
-template <int MODE, class Grid>
+template <int MODE, bool FUSE, class Grid>
 CRVPT_DEV void recordFirst(PathState& st, const SceneParams& P, const Grid& grid, float4* feat, V3 p, V3 w,
                            float pdfW, float dens, float depth) {
     if (!feat || (st.flags & PF_FIRST)) return;
     st.flags |= PF_FIRST;
-    const V3 n = cloudFiniteDifference(grid, P, st, p);
+    const V3 n = cloudFiniteDifference<FUSE>(grid, P, st, p);
     const size_t k = 3 * size_t(st.unit);
     feat[k] = make_float4(p.x, p.y, p.z, depth);
     feat[k + 1] = make_float4(w.x, w.y, w.z, pdfW);
@@ -476,7 +492,7 @@ CRVPT_DEV bool scatterEvent(PathState& st, Walker& W, const SceneParams& P, cons
         // ratio tracking records neither depth nor density (RatioTracking.glsl:75-81)
         const bool ratio = MODE == VPT_RATIO_TRACKING;
         const float ext = (isNee<MODE>() || isSpectral<MODE>()) ? P.extinctionMax : P.extinction;
-        recordFirst<MODE>(st, P, grid, feat, p, nw, evalPhase(P, W.w, nw), ratio ? 0.0f : rho * ext,
+        recordFirst<MODE, !isSpectral<MODE>()>(st, P, grid, feat, p, nw, evalPhase(P, W.w, nw), ratio ? 0.0f : rho * ext,
                           ratio ? 0.0f : W.t);
     }
     if (MODE == VPT_RATIO_TRACKING) st.thr *= 1.0f - pAbsOverReal;
@@ -600,7 +616,7 @@ CRVPT_DEV bool spectralCollision(PathState& st, Walker& W, const SceneParams& P,
     Ps /= C;
     Pn /= C;
     if (xi < Pa) {
-        recordFirst<MODE>(st, P, grid, feat, p, v3(0.0f), 0.0f, rho * P.extinctionMax, W.t);
+        recordFirst<MODE, false>(st, P, grid, feat, p, v3(0.0f), 0.0f, rho * P.extinctionMax, W.t);
         finishPath(st, isNee<MODE>() ? st.color : v3(0.0f), true);
         return false;
     }
@@ -635,7 +651,7 @@ CRVPT_DEV bool stepPath(PathState& st, Walker& W, const SceneParams& P, const Su
             st.flags |= PF_PENDING | PF_PEND_END;
             return true;
         }
-        const float rho = grid.lookupWorldJ(P, W.o + W.w * W.t, jitterHi(r.y), jitterLo(r.y), jitterHi(r.z), gc);
+        const float rho = tapDensity<MODE>(grid, P, W.o + W.w * W.t, r, gc);
         st.taps++;
         st.thr *= 1.0f - (P.extinction * rho - W.muC) * rcpf(W.mu);
         st.wSum += st.thr;
@@ -656,7 +672,7 @@ CRVPT_DEV bool stepPath(PathState& st, Walker& W, const SceneParams& P, const Su
         // control collision (xi * mu < mu_c) needs no lookup; a residual one is real with prob (sigma rho - mu_c)/mu_r
         const float xm = xi * W.mu;
         if (!(xm < W.muC)) {
-            const float rho = grid.lookupWorldJ(P, p, jitterHi(r.y), jitterLo(r.y), jitterHi(r.z), gc);
+            const float rho = tapDensity<MODE>(grid, P, p, r, gc);
             st.taps++;
             if (!(xm < P.extinction * rho)) return true;
         }
@@ -668,7 +684,7 @@ CRVPT_DEV bool stepPath(PathState& st, Walker& W, const SceneParams& P, const Su
         st.flags |= PF_PENDING;
         return true;
     }
-    const float rho = grid.lookupWorldJ(P, p, jitterHi(r.y), jitterLo(r.y), jitterHi(r.z), gc);
+    const float rho = tapDensity<MODE>(grid, P, p, r, gc);
     st.taps++;
     const float pReal = P.extinction * rho * rcpf(W.mu);
     if (isSpectral<MODE>() && !(st.flags & PF_SHADOW))
@@ -686,7 +702,7 @@ CRVPT_DEV bool stepPath(PathState& st, Walker& W, const SceneParams& P, const Su
         // absorption or a scattering event beyond the bounce limit: delta / ratio end with 0, next-event with its sum
         if (MODE != VPT_RATIO_TRACKING && xi < pAbs) {
             // delta tracking records w = 0 (DeltaTracking.glsl:291-300), next-event the incoming direction
-            recordFirst<MODE>(st, P, grid, feat, p, isNee<MODE>() ? W.w : v3(0.0f), 0.0f,
+            recordFirst<MODE, false>(st, P, grid, feat, p, isNee<MODE>() ? W.w : v3(0.0f), 0.0f,
                               rho * (isNee<MODE>() ? P.extinctionMax : P.extinction), W.t);
         }
         finishPath(st, isNee<MODE>() ? st.color : v3(0.0f), true);
