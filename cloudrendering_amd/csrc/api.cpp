@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/crvpt.h"
+#include "batch_plan.hpp"
 #include "host_common.hpp"
 #include "nanovdb_build.hpp"
 #include "parallel_for.hpp"
@@ -2101,21 +2102,20 @@ BatchLaunch resolvedLaunch(const Batch& b, const Renderer& r, BatchLaunch c) {
     return c;
 }
 
-// The launch of one render: units of fewer samples than configured where the batch is too small for them (a lane's unit
-// is a chain of samples, and a launch lasts as long as its last chain), one per 64 paths that a lane gets. 8 requests of
-// 6.6 M paths, 25 per lane: 90.3 / 57.1 / 47.7 ms with 16 / 4 / 1 samples per unit.
+// The launch of one render: the units cut to the batch's size.
 BatchLaunch renderLaunch(const Batch& b, BatchLaunch c) {
-    uint64_t paths = 0;
-    for (const BatchRequest& q : b.reqs) paths += uint64_t(q.P.width) * uint64_t(q.P.height) * q.spp;
-    const uint64_t perLane = paths / (uint64_t(c.numBlocks) * uint64_t(c.blockSize));
-    c.samplesPerUnit = uint32_t(std::min<uint64_t>(c.samplesPerUnit, std::max<uint64_t>(perLane / 64, 1)));
+    std::vector<BatchSize> sizes;
+    for (const BatchRequest& q : b.reqs) sizes.push_back({uint64_t(q.P.width) * uint64_t(q.P.height), q.spp});
+    c.samplesPerUnit = batchSamplesPerUnit(sizes.data(), sizes.size(), c.samplesPerUnit,
+                                           uint64_t(c.numBlocks) * uint64_t(c.blockSize));
     return c;
 }
 
-// Units of one sample leave the launch's last paths to the drain.
+// Units of one sample leave the launch's last paths to the drain (the table of units has been uploaded).
 int prepareBatchDrain(Batch& b, const BatchLaunch& c) {
     if (c.samplesPerUnit != 1u) return CRVPT_OK;
-    HIP_TRY(b.dDrain.ensure(size_t(c.numBlocks) * c.blockSize * kDrainWords * sizeof(uint32_t)));
+    const uint64_t states = batchDrainStates(b.totalUnits, uint64_t(c.numBlocks) * uint64_t(c.blockSize));
+    HIP_TRY(b.dDrain.ensure(std::max<uint64_t>(states, 1) * kDrainWords * sizeof(uint32_t)));
     return CRVPT_OK;
 }
 
