@@ -2097,18 +2097,22 @@ int uploadBatchTable(Batch& b, uint32_t samplesPerUnit) {
     return CRVPT_OK;
 }
 
-BatchLaunch resolvedLaunch(const Batch& b, const Renderer& r, BatchLaunch c) {
+// The launch of a render with a configuration: the workgroups of 0 by occupancy, the units cut to the batch's size. spp:
+// the requests' sample counts where the batch's own are reduced (autotuner).
+BatchLaunch renderLaunch(const Batch& b, const Renderer& r, BatchLaunch c, const std::vector<uint32_t>* spp = nullptr) {
     if (c.numBlocks == 0) c.numBlocks = uint32_t(r.cuCount * batchOccupancyBlocksPerCU(b.mode, c.blockSize));
+    std::vector<BatchSize> sizes;
+    for (size_t i = 0; i < b.reqs.size(); i++)
+        sizes.push_back({uint64_t(b.reqs[i].P.width) * uint64_t(b.reqs[i].P.height), spp ? (*spp)[i] : b.reqs[i].spp});
+    if (!sizes.empty())
+        c.samplesPerUnit = batchSamplesPerUnit(sizes.data(), sizes.size(), c.samplesPerUnit,
+                                               uint64_t(c.numBlocks) * uint64_t(c.blockSize));
     return c;
 }
 
-// The launch of one render: the units cut to the batch's size.
-BatchLaunch renderLaunch(const Batch& b, BatchLaunch c) {
-    std::vector<BatchSize> sizes;
-    for (const BatchRequest& q : b.reqs) sizes.push_back({uint64_t(q.P.width) * uint64_t(q.P.height), q.spp});
-    c.samplesPerUnit = batchSamplesPerUnit(sizes.data(), sizes.size(), c.samplesPerUnit,
-                                           uint64_t(c.numBlocks) * uint64_t(c.blockSize));
-    return c;
+bool sameLaunch(const BatchLaunch& a, const BatchLaunch& b) {
+    return a.numBlocks == b.numBlocks && a.blockSize == b.blockSize && a.stepsPerRefill == b.stepsPerRefill &&
+           a.samplesPerUnit == b.samplesPerUnit;
 }
 
 // Units of one sample leave the launch's last paths to the drain (the table of units has been uploaded).
@@ -2221,11 +2225,11 @@ int crvpt_batch_get_launch_config(int32_t config[4]) {
     if (int rc = requireBatch()) return rc;
     if (!config) return fail(CRVPT_ERR_INVALID_ARGUMENT, "batch_get_launch_config: null output");
     Batch& b = *g_batch;
-    const BatchLaunch c = b.mode >= 0 ? resolvedLaunch(b, *g_r, b.blocksAuto ? BatchLaunch{0, b.cfg.blockSize,
-                                                                                          b.cfg.stepsPerRefill,
-                                                                                          b.cfg.samplesPerUnit}
-                                                                         : b.cfg)
-                                      : b.cfg;
+    BatchLaunch c = b.cfg;
+    if (b.mode >= 0) {
+        if (b.blocksAuto) c.numBlocks = 0;
+        c = renderLaunch(b, *g_r, c);
+    }
     config[0] = int32_t(c.numBlocks);
     config[1] = c.blockSize;
     config[2] = c.stepsPerRefill;
@@ -2241,7 +2245,7 @@ int crvpt_batch_render(uint32_t frame_offset, void* stream) {
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     BatchLaunch c = b.cfg;
     if (b.blocksAuto) c.numBlocks = 0;
-    c = renderLaunch(b, resolvedLaunch(b, r, c));
+    c = renderLaunch(b, r, c);
     if (b.tableDirty) {
         HIP_TRY(hipDeviceSynchronize());  // a previous launch may still read the table
         if (int rc = uploadBatchTable(b, c.samplesPerUnit)) return rc;
@@ -2310,8 +2314,8 @@ int crvpt_batch_autotune(int spp_divisor, int32_t config[4]) {
         for (size_t i = 0; i < b.reqs.size(); i++) b.reqs[i].spp = spp[i];
         b.tableDirty = true;
     };
-    auto timeConfig = [&](BatchLaunch c, double& best) -> int {
-        c = resolvedLaunch(b, r, c);
+    // c: a launch as batch_render makes it, its units cut for the full sample counts
+    auto timeLaunch = [&](const BatchLaunch& c, double& best) -> int {
         if (int rc = uploadBatchTable(b, c.samplesPerUnit)) return rc;
         if (int rc = prepareBatchDrain(b, c)) return rc;
         HIP_TRY(launchSetU32(b.dFrame.as<uint32_t>(), 0u, s));
@@ -2330,19 +2334,24 @@ int crvpt_batch_autotune(int spp_divisor, int32_t config[4]) {
     };
     // Coordinate descent from the current configuration: compaction interval, paths per unit, block size, then the
     // number of persistent workgroups as a fraction of the occupancy limit.
+    // Different settings of the samples per unit can come to one launch, which is timed once.
     BatchLaunch cur = b.cfg;
     cur.numBlocks = 0;
+    BatchLaunch curLaunch = renderLaunch(b, r, cur, &spp);
     double curMs = 0.0;
-    if (int rc = timeConfig(cur, curMs)) {
+    if (int rc = timeLaunch(curLaunch, curMs)) {
         restore();
         return rc;
     }
-    auto tryConfig = [&](BatchLaunch c) -> int {
+    auto tryConfig = [&](const BatchLaunch& c) -> int {
+        const BatchLaunch l = renderLaunch(b, r, c, &spp);
+        if (sameLaunch(l, curLaunch)) return CRVPT_OK;
         double ms = 0.0;
-        if (int rc = timeConfig(c, ms)) return rc;
+        if (int rc = timeLaunch(l, ms)) return rc;
         if (ms < curMs) {
             curMs = ms;
             cur = c;
+            curLaunch = l;
         }
         return CRVPT_OK;
     };
@@ -2363,7 +2372,7 @@ int crvpt_batch_autotune(int spp_divisor, int32_t config[4]) {
     for (int bs : {64, 128, 256})
         if (!rc && bs != cur.blockSize) rc = tryConfig(BatchLaunch{0, bs, cur.stepsPerRefill, cur.samplesPerUnit});
     if (!rc) {
-        const uint32_t full = resolvedLaunch(b, r, BatchLaunch{0, cur.blockSize, 1, 1}).numBlocks;
+        const uint32_t full = renderLaunch(b, r, BatchLaunch{0, cur.blockSize, 1, 1}, &spp).numBlocks;
         for (int num : {1, 2})
             if (!rc) rc = tryConfig(BatchLaunch{std::max(1u, full * uint32_t(num) / 3u), cur.blockSize,
                                                 cur.stepsPerRefill, cur.samplesPerUnit});
@@ -2373,7 +2382,7 @@ int crvpt_batch_autotune(int spp_divisor, int32_t config[4]) {
     b.cfg = cur;
     b.blocksAuto = cur.numBlocks == 0;
     if (config) {
-        const BatchLaunch c = resolvedLaunch(b, r, cur);
+        const BatchLaunch c = renderLaunch(b, r, cur);
         config[0] = int32_t(c.numBlocks);
         config[1] = c.blockSize;
         config[2] = c.stepsPerRefill;

@@ -285,6 +285,8 @@ int crvpt_batch_render(uint32_t frame_offset, void* stream);
  * walker steps between refills (compaction interval), samples per claimed unit (paths per lane; an upper bound, a
  * batch with few units per lane takes fewer)}. */
 int crvpt_batch_set_launch_config(int blocks, int block_size, int steps_per_refill, int samples_per_unit);
+/* The configuration; once the batch holds a request, as crvpt_batch_render runs it: the workgroups in place of 0 and the
+ * samples per unit that the batch's size leaves. */
 int crvpt_batch_get_launch_config(int32_t config[4]);
 /* Times candidate launch configurations on the batch with spp / spp_divisor samples per request (coordinate descent
  * over the compaction interval, samples per unit, block size and workgroup count), keeps the fastest and returns it
