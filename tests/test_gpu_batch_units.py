@@ -58,3 +58,24 @@ def test_autotune_keeps_a_launch_that_renders(vpt):
     for a, b in zip(tuned, vpt.batch_render()):
         assert bool((a == b).all())
     vpt.batch_clear()
+
+
+@pytest.mark.parametrize("samples", [2, 3, 16])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4, 5, 6])
+def test_units_of_several_samples_trace_the_same_paths(vpt, mode, samples):
+    """One workgroup of 64 lanes keeps `samples` per unit (17 samples per pixel: the last unit of a pixel is a part);
+    units of one sample leave their last paths to the drain. Equal up to the float sum within a unit: non-negative
+    samples, so samples - 1 roundings of 2^-24 and one more of each result."""
+    import numpy as np
+
+    print(f"case: batch units mode={mode} samples={samples}", flush=True)
+    _batch(vpt, mode, 48, 17)
+    vpt.batch_set_launch_config(0, 256, 16, 1)
+    want = [o.cpu().numpy().astype(np.float64) for o in vpt.batch_render()]
+    vpt.batch_set_launch_config(1, 64, 16, samples)
+    assert vpt.batch_get_launch_config()["samples_per_unit"] == samples
+    for k, (a, b) in enumerate(zip(vpt.batch_render(), want)):
+        a = a.cpu().numpy().astype(np.float64)
+        off = np.abs(a - b) > (samples + 1) * 2.0 ** -24 * b
+        assert not off.any(), f"request {k}: {int(off.sum())} of {off.size} values differ"
+    vpt.batch_clear()
