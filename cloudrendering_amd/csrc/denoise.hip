@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "render_api.hpp"
+#include "rounded.hpp"
 
 namespace crvpt {
 
@@ -117,18 +118,25 @@ __device__ __forceinline__ float fetchW(const float4* img, int x, int y, int w, 
     return inImage(x, y, w, h) ? img[size_t(y) * w + x].w : 0.0f;
 }
 
-// compute_weight (svgf_common.glsl): sigma_n = 128; fmaxf keeps the non-NaN operand like GLSL max on the GPU. rPhiD, rPhiC:
-// 1 / phi_depth and 2 / phi_colour, divided once per pixel (and tap distance) instead of twice per tap. The 128th power is
-// seven squarings in FP64 (correctly rounded to float but for a 2^-46 chance); the library's powf took half the time of
-// both filters.
-__device__ __forceinline__ float svgfWeight(float4 cg, float4 og, float rPhiD, float cc, float oc, float rPhiC) {
+// A divisor and its rounded reciprocal, divided once per pixel (and tap distance) for all taps.
+struct SvgfScale {
+    float phi, r;
+    __device__ __forceinline__ explicit SvgfScale(float p) : phi(p), r(1.0f / p) {}
+    SvgfScale() = default;
+};
+
+// compute_weight (svgf_common.glsl): sigma_n = 128; fmaxf keeps the non-NaN operand like GLSL max on the GPU. The
+// quotients are the divisions' (quotient). The 128th power is seven squarings in FP64: the first is exact, the other six
+// leave a relative error below 2^-46 before the rounding to float, which then misses the nearest in about one of 2^22
+// taps; the library's powf took half the time of both filters.
+__device__ __forceinline__ float svgfWeight(float4 cg, float4 og, SvgfScale depth, float cc, float oc, SvgfScale color) {
     const float d = fmaxf(0.0f, cg.x * og.x + cg.y * og.y + cg.z * og.z);
     double p = double(d);
 #pragma unroll
     for (int k = 0; k < 7; k++) p *= p;
     const float wn = float(p);
-    const float wz = fabsf(cg.w - og.w) * rPhiD;
-    const float wc = fabsf(cc - oc) * rPhiC;
+    const float wz = quotient(fabsf(cg.w - og.w), depth.phi, depth.r);
+    const float wc = quotient(fabsf(cc - oc) * 2.0f, color.phi, color.r);
     return __expf(0.0f - fmaxf(wc, 0.0f) - fmaxf(wz, 0.0f)) * wn;
 }
 
@@ -237,7 +245,7 @@ __global__ void k_svgfReproject(SvgfFrame F, float4* __restrict__ accumMoments, 
 // Compute-Filter-Moments: 7x7 cross-bilateral estimate of the variance while the history is short (< 4 frames). Also
 // keeps the frame's guide and moments as the next frame's history (the reprojection, which reads the old ones, is done).
 // A workgroup with a short history stages its 16 x 16 pixels' taps, 22 x 22, in LDS: colour and first moment, guide and
-// second moment, 36 B per tap. 1280 x 720, 49 taps: 217 us with four 16-byte loads and a powf per tap, now 46 us.
+// second moment, 36 B per tap. 1280 x 720, 49 taps: 217 us with four 16-byte loads and a powf per tap, now 51 us.
 constexpr int kMomentHalo = 16 + 6;
 
 __global__ __launch_bounds__(256) void k_svgfFilterMoments(SvgfFrame F, const float4* __restrict__ accumMoments,
@@ -286,7 +294,7 @@ __global__ __launch_bounds__(256) void k_svgfFilterMoments(SvgfFrame F, const fl
         tempOut[i] = tempIn[i];
         return;
     }
-    const float rPhiD = 1.0f / (fabsf(F.depth[i].w) + 0.0001f), rPhiC = 2.0f / 10.0f;
+    const SvgfScale phiD(fabsf(F.depth[i].w) + 0.0001f), phiC(10.0f);
     const float cc = tempIn[i].x;
     float sw = 0.0f;
     float3 sc = make_float3(0.0f, 0.0f, 0.0f);
@@ -297,7 +305,7 @@ __global__ __launch_bounds__(256) void k_svgfFilterMoments(SvgfFrame F, const fl
             if (!inImage(x + xx, y + yy, F.w, F.h)) continue;
             const int e = (int(threadIdx.y) + 3 + yy) * kMomentHalo + int(threadIdx.x) + 3 + xx;
             const float4 oc = tc[e];
-            const float wt = svgfWeight(cg, tg[e], rPhiD, cc, oc.x, rPhiC);
+            const float wt = svgfWeight(cg, tg[e], phiD, cc, oc.x, phiC);
             sw += wt;
             sc = make_float3(sc.x + wt * oc.x, sc.y + wt * oc.y, sc.z + wt * oc.z);
             sm = make_float2(sm.x + wt * oc.w, sm.y + wt * tm[e]);
@@ -312,8 +320,8 @@ __global__ __launch_bounds__(256) void k_svgfFilterMoments(SvgfFrame F, const fl
 
 // Compute-ATrous iteration `it` (step 2^it): 5x5 kernel (1, 2/3, 1/6), colour scale from the 3x3-blurred variance,
 // the variance channel weighted by squared weights. Bound by the taps' loads: colour and guide of a row of five taps are
-// loaded before any is used, at addresses clamped into the image (taps outside it weigh 0 and add 0), instead of three
-// loads behind each tap's own branch. 1280 x 720: 125 -> 42 us per iteration (96 us with the library powf in the weight).
+// loaded before any is used, at addresses clamped into the image (taps outside it are skipped), instead of three loads
+// behind each tap's own branch. 1280 x 720: 125 -> 44 us per iteration (96 us with the library powf in the weight).
 __global__ __launch_bounds__(256) void k_svgfAtrous(SvgfFrame F, const float4* __restrict__ color,
                                                     float4* __restrict__ out, float4* __restrict__ history, int it) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y;
@@ -327,7 +335,7 @@ __global__ __launch_bounds__(256) void k_svgfAtrous(SvgfFrame F, const float4* _
     for (int yy = -1; yy <= 1; yy++)
 #pragma unroll
         for (int xx = -1; xx <= 1; xx++) fv += fetchW(color, x + xx, y + yy, F.w, F.h) * kg[abs(xx)][abs(yy)];
-    const float rPhiC = 2.0f / sqrtf(fmaxf(0.0f, 1e-10f + fv));
+    const SvgfScale phiC(sqrtf(fmaxf(0.0f, 1e-10f + fv)));
     const float4 c0 = color[i];
     const float4 cg = F.guide[i];
     const float cf = F.depth[i].w;
@@ -339,10 +347,10 @@ __global__ __launch_bounds__(256) void k_svgfAtrous(SvgfFrame F, const float4* _
         const float4* crow = color + size_t(qy) * F.w;
         const float4* grow = F.guide + size_t(qy) * F.w;
         const float ky = yy == 0 ? kv[0] : (yy == 1 || yy == -1 ? kv[1] : kv[2]);
-        float rPhiD[3];  // by |xx|
+        SvgfScale phiD[3];  // by |xx|
 #pragma unroll
         for (int a = 0; a < 3; a++)
-            rPhiD[a] = 1.0f / (fabsf(cf * sqrtf(float(a * a + yy * yy)) * float(step)) + 0.0001f);
+            phiD[a] = SvgfScale(fabsf(cf * sqrtf(float(a * a + yy * yy)) * float(step)) + 0.0001f);
         float4 oc[5], og[5];
 #pragma unroll
         for (int xx = 0; xx < 5; xx++) {
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(256) void k_svgfAtrous(SvgfFrame F, const float4* _
             const int qx = x + (xx - 2) * step;
             if (qx < 0 || qx >= F.w || (xx == 2 && yy == 0)) continue;
             const int ax = xx < 2 ? 2 - xx : xx - 2;
-            const float wt = svgfWeight(cg, og[xx], rPhiD[ax], c0.x, oc[xx].x, rPhiC) * (kv[ax] * ky);
+            const float wt = svgfWeight(cg, og[xx], phiD[ax], c0.x, oc[xx].x, phiC) * (kv[ax] * ky);
             sum = make_float4(sum.x + wt * oc[xx].x, sum.y + wt * oc[xx].y, sum.z + wt * oc[xx].z,
                               sum.w + wt * wt * oc[xx].w);
             acc += wt;
