@@ -30,13 +30,13 @@ constexpr int kConvBlocksPerCU = 2;
 
 struct KpnModel {
     DevBuf params, grads, m1, m2, wFwd, wBwd, loss;
-    DevBuf act, logits, dzA, dzB, last, gradWork;
+    DevBuf act, dzA, dzB, last, gradWork;
     size_t capPixels = 0;
     int step = 0;
     bool ready = false;
     int cuCount = 256;
     ~KpnModel() {
-        for (DevBuf* b : {&params, &grads, &m1, &m2, &wFwd, &wBwd, &loss, &act, &logits, &dzA, &dzB, &last, &gradWork})
+        for (DevBuf* b : {&params, &grads, &m1, &m2, &wFwd, &wBwd, &loss, &act, &dzA, &dzB, &last, &gradWork})
             b->release();
     }
 };
@@ -92,7 +92,6 @@ int ensureActivations(size_t P) {
     const size_t bf = P * kKpnChannels * 2;
     k.capPixels = 0;  // a failed allocation leaves no pass or logits to run on the released buffers
     HIP_TRY(k.act.ensure(bf * kKpnLayers));  // inputs of the six layers
-    HIP_TRY(k.logits.ensure(P * kKpnChannels * sizeof(float)));
     HIP_TRY(k.dzA.ensure(bf));
     HIP_TRY(k.dzB.ensure(bf));
     k.capPixels = P;
@@ -256,8 +255,7 @@ int crvpt_kpn_get_logits(float* out, int n, int h, int w, void* stream) {
     if (!out || P == 0 || P > k.capPixels) return fail(CRVPT_ERR_INVALID_ARGUMENT, "kpn_get_logits: bad shape");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     // the forward pass keeps its logits in LDS: its last layer runs again, on the input and weights it had
-    HIP_TRY(launchKpnLogits(k.act.ptr, k.last.ptr, k.logits.as<float>(), k.cuCount * kConvBlocksPerCU, s));
-    HIP_TRY(hipMemcpyAsync(out, k.logits.ptr, P * kKpnChannels * sizeof(float), hipMemcpyDeviceToDevice, s));
+    HIP_TRY(launchKpnLogits(k.act.ptr, k.last.ptr, out, P, k.cuCount * kConvBlocksPerCU, s));
     return CRVPT_OK;
 }
 

@@ -159,19 +159,18 @@ __device__ __forceinline__ void loadBias(const float* __restrict__ bias, int kb,
 template <int EPI>
 __device__ __forceinline__ void storeTile(const f32x4 (&acc)[4][2], const float (&bco)[2][4],
                                           const __bf16* __restrict__ mask, void* __restrict__ out, int n, int H, int W,
-                                          int yw, int x, int kb) {
+                                          int yw, int x, int kb, size_t outPixels) {
 #pragma unroll
     for (int mt = 0; mt < 4; mt++) {
         const int y = yw + mt;
         if (y >= H || x >= W) continue;
         const size_t o = ((size_t(n) * H + y) * W + x) * kC + kb * 8;
         if (EPI == EPI_LINEAR_F32) {
+            // a caller's buffer: of any float alignment, and of outPixels pixels
+            if (o >= outPixels * kC) continue;
+            float* dst = reinterpret_cast<float*>(out) + o;
 #pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                const f32x4 v = acc[mt][nt];
-                reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + o)[nt] =
-                    make_float4(v[0] + bco[nt][0], v[1] + bco[nt][1], v[2] + bco[nt][2], v[3] + bco[nt][3]);
-            }
+            for (int i = 0; i < 8; i++) dst[i] = acc[mt][i >> 2][i & 3] + bco[i >> 2][i & 3];
         } else {
             bf16x8 r;
             if (EPI == EPI_RELU_BF16) {
@@ -201,7 +200,7 @@ __device__ __forceinline__ void storeTile(const f32x4 (&acc)[4][2], const float 
 template <int EPI, int CIN = kC>
 __device__ __forceinline__ void convLayer(const __bf16* __restrict__ in, const bf16x8* __restrict__ wsw,
                                           const float* __restrict__ bias, const __bf16* __restrict__ mask,
-                                          void* __restrict__ out, int N, int H, int W) {
+                                          void* __restrict__ out, int N, int H, int W, size_t outPixels = 0) {
     __shared__ __attribute__((aligned(16))) __bf16 tile[kHalo * kHalo * kPixStride];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, kb = lane >> 4;
@@ -222,7 +221,7 @@ __device__ __forceinline__ void convLayer(const __bf16* __restrict__ in, const b
         if (walk.valid()) halo.load(in, walk.n, H, W, walk.y0, walk.x0);
         f32x4 acc[4][2];
         convTaps<EPI == EPI_MASK_BF16>(tile, B, wave, m, kb, acc);
-        storeTile<EPI>(acc, bco, mask, out, n, H, W, y0 + wave * 4, x0 + m, kb);
+        storeTile<EPI>(acc, bco, mask, out, n, H, W, y0 + wave * 4, x0 + m, kb, outPixels);
     }
 }
 
@@ -433,12 +432,17 @@ __global__ __launch_bounds__(256, 2) void k_convHead(const __bf16* __restrict__ 
 }
 
 // The last forward pass's logits [N, H, W, 32] f32, from the final layer's input (the last of kKpnLayers activation
-// buffers of N * H * W pixels each at `act`) and the weights it ran with.
+// buffers of N * H * W pixels each at `act`) and the weights it ran with, into a caller's buffer of outPixels pixels:
+// what is beyond it is left out, pixels of it beyond the pass are 0.
 __global__ __launch_bounds__(256) void k_convLogits(const __bf16* __restrict__ act,
-                                                    const KpnLastForward* __restrict__ last, float* __restrict__ out) {
+                                                    const KpnLastForward* __restrict__ last, float* __restrict__ out,
+                                                    size_t outPixels) {
     const int N = last->N, H = last->H, W = last->W;
-    convLayer<EPI_LINEAR_F32>(act + size_t(kKpnLayers - 1) * N * H * W * kC, last->frag, last->bias, nullptr, out, N, H,
-                              W);
+    const size_t P = size_t(N) * H * W, first = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    for (size_t i = P * kC + first; i < outPixels * kC; i += size_t(gridDim.x) * blockDim.x) out[i] = 0.0f;
+    if (P == 0) return;
+    convLayer<EPI_LINEAR_F32>(act + size_t(kKpnLayers - 1) * P * kC, last->frag, last->bias, nullptr, out, N, H, W,
+                              outPixels);
 }
 
 // Weight and bias gradients of one layer: dW[co][ci][tap] = sum over pixels p of dZ[p][co] * X[p + offset(tap)][ci] and
@@ -704,9 +708,11 @@ hipError_t launchKpnConvHead(const void* in, const void* wsw, const float* bias,
     return hipGetLastError();
 }
 
-hipError_t launchKpnLogits(const void* act, const void* last, float* out, int blocks, hipStream_t stream) {
+hipError_t launchKpnLogits(const void* act, const void* last, float* out, size_t outPixels, int blocks,
+                           hipStream_t stream) {
     hipLaunchKernelGGL(k_convLogits, dim3(unsigned(blocks)), dim3(256), 0, stream,
-                       reinterpret_cast<const __bf16*>(act), reinterpret_cast<const KpnLastForward*>(last), out);
+                       reinterpret_cast<const __bf16*>(act), reinterpret_cast<const KpnLastForward*>(last), out,
+                       outPixels);
     return hipGetLastError();
 }
 

@@ -103,7 +103,8 @@ constexpr size_t kKpnLastForwardBytes = 32 * 1024;
 hipError_t launchKpnConvHead(const void* in, const void* wsw, const float* bias, const float* noisy,
                              const float* target, float* pred, void* dz, float* loss, void* last, int N, int H, int W,
                              int blocks, hipStream_t stream);
-hipError_t launchKpnLogits(const void* act, const void* last, float* out, int blocks, hipStream_t stream);
+hipError_t launchKpnLogits(const void* act, const void* last, float* out, size_t outPixels, int blocks,
+                           hipStream_t stream);
 // Partial sums of one layer's weight and bias gradients, then the gradients of all layers from them; work:
 // kpnGradWorkFloats(blocks) floats, blocks: workgroups (rows of partial sums) per layer.
 size_t kpnGradWorkFloats(int blocks);

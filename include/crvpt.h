@@ -261,7 +261,8 @@ int crvpt_kpn_adam_step(float lr, void* stream);
 int crvpt_kpn_train_step(const float* features, const float* noisy, const float* target, int n, int h, int w,
                          float lr, float* loss, void* stream);
 int crvpt_kpn_denoise(const float* features, const float* noisy, float* out, int n, int h, int w, void* stream);
-/* Logits [n, h, w, 32] f32 of the last forward pass (channels 25..31 are padding). */
+/* Logits [n, h, w, 32] f32 of the last forward pass (channels 25..31 are padding), recomputed by its last layer into out;
+ * pixels beyond those of the pass are 0. */
 int crvpt_kpn_get_logits(float* out, int n, int h, int w, void* stream);
 int crvpt_kpn_release(void);
 
