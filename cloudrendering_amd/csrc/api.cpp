@@ -1802,14 +1802,22 @@ int crvpt_transmittance_batch(int estimator, int n_rays, const float* origins, c
     }
     HIP_TRY(hipEventRecord(r.ev0, s));
     // the estimates of several samples per ray share one buffer: a call on another stream waits for the last one's
-    const size_t work = transmittanceWorkBytes(n_rays, n_samples);
-    if (work > 0) {
-        HIP_TRY(r.dTrans.ensure(work));
+    TransmittancePlan plan = transmittancePlan(n_rays, n_samples, kTransmittanceUnits);
+    if (plan.bytes() > 0) {
+        hipError_t e = r.dTrans.ensure(plan.bytes());
+        // where memory is short: smaller launches, down to half a megabyte of estimates
+        for (size_t units = kTransmittanceUnits / 8; e == hipErrorOutOfMemory && units >= kTransmittanceUnitsMin;
+             units /= 8) {
+            (void)hipGetLastError();
+            plan = transmittancePlan(n_rays, n_samples, units);
+            e = r.dTrans.ensure(plan.bytes());
+        }
+        HIP_TRY(e);
         HIP_TRY(hipStreamWaitEvent(s, r.evTrans, 0));
     }
     HIP_TRY(launchTransmittance(P, sp ? nullptr : &dg, sp ? &ng : nullptr, S, estimator, o, d, tm, n_rays, n_samples,
-                                seed, mo, m2o, r.dTrans.ptr, r.cuCount, s));
-    if (work > 0) HIP_TRY(hipEventRecord(r.evTrans, s));
+                                seed, mo, m2o, plan, r.dTrans.ptr, r.cuCount, s));
+    if (plan.bytes() > 0) HIP_TRY(hipEventRecord(r.evTrans, s));
     HIP_TRY(hipEventRecord(r.ev1, s));
     HIP_TRY(hipEventRecord(r.evT1, s));
     if (!on_device) {

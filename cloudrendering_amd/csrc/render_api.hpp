@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "transmittance_plan.hpp"
 #include "vpt_types.h"
 
 namespace crvpt {
@@ -129,13 +130,11 @@ hipError_t launchAccumulateFeatures(const SceneParams& P, const float4* paths, c
 // Writes feature map `map` (FeatureMapTypeVpt order) as C planes of H*W floats; result = the image accumulator.
 hipError_t launchFeatureOut(int map, const FeatureAcc& acc, const float4* result, uint32_t npix, float* outCHW,
                             int channels, hipStream_t stream);
-// Batched transmittance queries (transmittance.hip). work: transmittanceWorkBytes of device memory (none for one sample).
-constexpr size_t kTransmittanceUnits = size_t(1) << 26;  // estimates per launch
-size_t transmittanceWorkBytes(int nRays, int nSamples);
+// Batched transmittance queries (transmittance.hip). work: plan.bytes() of device memory.
 hipError_t launchTransmittance(const SceneParams& P, const DenseGrid* dense, const NanoGrid* nano,
                                const SupervoxelGrid& S, int estimator, const float* o, const float* d,
                                const float* tmax, int nRays, int nSamples, uint32_t seed, float* mean, float* m2,
-                               void* work, int cuCount, hipStream_t stream);
+                               const TransmittancePlan& plan, void* work, int cuCount, hipStream_t stream);
 // Flat 8^3-block index of a NanoVDB grid over blocks [b0, b0 + nb) (see NanoGrid::blockLeaf); *bad (cleared by the
 // caller) becomes nonzero when a leaf offset cannot be encoded.
 hipError_t launchBlockTable(const NanoGrid& nano, const int b0[3], const int nb[3], uint32_t* leaf, float* tile,

@@ -299,8 +299,8 @@ __global__ __launch_bounds__(256) void k_transmittanceTable(SceneParams P, Grid 
     }
 }
 
-// Sums of a launch's estimates per ray, in sample order; sums (nullable on the only launch of a ray) carries them from
-// one launch of a ray's samples to the next.
+// Sums of a launch's estimates per ray, in sample order; sums (null where every ray's samples are in one launch) carries
+// them from one launch of a ray's samples to the next.
 __global__ void k_transmittanceMean(const float* __restrict__ records, RayBatch B, double2* __restrict__ sums,
                                     float* __restrict__ mean, float* __restrict__ m2) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -348,23 +348,15 @@ static void launchWalk(const SceneParams& P, const Grid& grid, const SupervoxelG
     }
 }
 
-size_t transmittanceWorkBytes(int nRays, int nSamples) {
-    if (nSamples <= 1) return 0;
-    const size_t samples = std::min(size_t(nSamples), kTransmittanceUnits);
-    const size_t rays = std::min(size_t(nRays), std::max<size_t>(1, kTransmittanceUnits / samples));
-    return rays * sizeof(double2) + rays * samples * sizeof(float);
-}
-
 hipError_t launchTransmittance(const SceneParams& P, const DenseGrid* dense, const NanoGrid* nano,
                                const SupervoxelGrid& S, int estimator, const float* o, const float* d,
                                const float* tmax, int nRays, int nSamples, uint32_t seed, float* mean, float* m2,
-                               void* work, int cuCount, hipStream_t stream) {
-    // a launch takes kTransmittanceUnits units at most: as many rays with all their samples as fit, or a part of one
-    // ray's samples
-    const size_t samples = std::min(size_t(nSamples), kTransmittanceUnits);
-    const size_t rays = std::min(size_t(nRays), std::max<size_t>(1, kTransmittanceUnits / samples));
-    double2* sums = reinterpret_cast<double2*>(work);
-    float* records = nSamples > 1 ? reinterpret_cast<float*>(sums + rays) : nullptr;
+                               const TransmittancePlan& plan, void* work, int cuCount, hipStream_t stream) {
+    const size_t samples = plan.samples, rays = plan.rays;
+    double2* sums = plan.sumBytes > 0 ? reinterpret_cast<double2*>(work) : nullptr;
+    float* records = plan.recordBytes > 0
+                             ? reinterpret_cast<float*>(reinterpret_cast<char*>(work) + plan.sumBytes)
+                             : nullptr;
     const RayResult out{mean, m2, records};
     const bool tri = P.interpolation == INTERP_TRILINEAR;
     for (size_t r0 = 0; r0 < size_t(nRays); r0 += rays)
