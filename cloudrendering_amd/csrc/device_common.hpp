@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rounded.hpp"
 #include "vpt_types.h"
 
 namespace crvpt {
@@ -151,20 +152,12 @@ CRVPT_DEV float evalPhase(const SceneParams& P, V3 a, V3 b) { return hgPdf(P, do
 // ------------------------------------------------------------------------------------------------------------
 // Sky and lights (VptUtils.glsl:271-453)
 // ------------------------------------------------------------------------------------------------------------
-// a / c from rc, the rounded 1 / c, with one correction: the correctly rounded quotient for the constant divisors used
-// here (checked over all mantissas on the host).
-CRVPT_DEV float divRounded(float a, float c, float rc) {
-    const float q = a * rc;
-    return fmaf(fmaf(-q, c, a), rc, q);
-}
-// x^2.4 for x in [2^-4, 2]: x^0.4 from the hardware log2 and exp2, one Newton step of y^5 = x^2 in FP64 (0.5001 units in
-// the last place of the exact power, against 1 for the library's power of the rounded exponent).
+// x^2.4 for x in [2^-4, 2] (pow24From).
 CRVPT_DEV float pow24(float x) {
     const double y = double(__builtin_amdgcn_exp2f(0.4f * __builtin_amdgcn_logf(x)));
     const double x2 = double(x) * double(x);
     const double y2 = y * y, y4 = y2 * y2;
-    const float d = float(fma(-y4, y, x2)) * __builtin_amdgcn_rcpf(5.0f * float(y4));
-    return float(x2 * (y + double(d)));
+    return pow24From(x2, y, y4, __builtin_amdgcn_rcpf(5.0f * float(y4)));
 }
 // LIBPOW: with the library's power. Every path that leaves the medium by the default sky takes three powers, and the
 // library's takes about three times the instructions of pow24: 1024^2 x 16 delta tracking of the 512^3 sparse grid

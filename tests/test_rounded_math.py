@@ -54,3 +54,57 @@ int main() {
     return bad != 0;
 }
 ''')
+
+
+def test_sky_divisions_are_exact(tmp_path):
+    """Every mantissa over each divisor of the default sky: the segments' widths and the two of the sRGB curve."""
+    _run(tmp_path, r'''
+int main() {
+    const float stops[] = {-1.0f, -0.1f, 0.0f, 0.4f, 1.0f};
+    float div[] = {12.92f, 1.055f, 0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 4; i++) div[2 + i] = stops[i + 1] - stops[i];
+    long bad = 0;
+    for (float c : div) {
+        const float rc = 1.0f / c;
+        for (uint32_t m = 0; m < (1u << 23); m++) {
+            const uint32_t bits = 0x3f800000u | m;
+            float a;
+            std::memcpy(&a, &bits, 4);
+            bad += divRounded(a, c, rc) != a / c;
+        }
+        for (float a : {0.0f, -0.0f, -0.7f, 2.0f, 1e-20f}) bad += divRounded(a, c, rc) != a / c;
+    }
+    std::printf("%ld mismatches\n", bad);
+    return bad != 0;
+}
+''')
+
+
+def test_power_2_4(tmp_path):
+    """Start values up to two units of float and reciprocals up to one unit off, as the hardware's exp2, log2 and rcp
+    give them, against the power in long double. Bound: half a unit from the last rounding; the start's relative error e
+    of 2^-22 leaves 2 e^2 = 2^-43 after the step, the float correction's own rounding e 2^-22 = 2^-44: 2^-18 units."""
+    _run(tmp_path, r'''
+int main() {
+    std::mt19937 g(3);
+    double worst = 0.0;
+    auto one = [&](float x) {
+        for (int off = -2; off <= 2; off++) {
+            float y = float(powl((long double)x, 0.4L));
+            for (int k = 0; k < (off < 0 ? -off : off); k++) y = nextafterf(y, off < 0 ? 0.0f : 2.0f);
+            const double yd = y, y4 = (yd * yd) * (yd * yd);
+            float r = 1.0f / (5.0f * float(y4));
+            if (off & 1) r = nextafterf(r, 0.0f);
+            const float p = pow24From(double(x) * double(x), yd, y4, r);
+            const long double want = powl((long double)x, 2.4L);
+            const double ulp = std::ldexp(1.0, std::ilogb(double(want)) - 23);
+            const double e = double(fabsl((long double)p - want)) / ulp;
+            if (e > worst) worst = e;
+        }
+    };
+    for (int i = 0; i < 400000; i++) one(0.0625f + 1.9375f * float(g() >> 8) * (1.0f / 16777216.0f));
+    for (float x : {0.0625f, 0.0904f, 1.0f, 0.99999994f, 2.0f}) one(x);
+    std::printf("worst %f units\n", worst);
+    return !(worst <= 0.501);
+}
+''')
