@@ -49,9 +49,20 @@ C2 = {"max_bounces": 128, "grid": 512, "edge0": 0.645, "edge1": 0.795, "width": 
       "modes": [(0, "delta tracking"), (2, "ratio tracking"), (4, "residual ratio tracking"),
                 (3, "decomposition tracking")], "gs": [0.0, 0.5, 0.85]}
 C1 = {"max_bounces": 64, "grid": 128, "width": 256, "height": 256, "spp": 64}
-MODE_KERNELS = {0: "k_pathPool<DELTA_TRACKING, NanoAccessT<false, false>, false, true>", 2: "k_pathPool<RATIO_TRACKING, NanoAccessT<false, false>, false, true>",
-                4: "k_pathPool<RESIDUAL_RATIO_TRACKING, NanoAccessT<false, false>, false, false>",
-                3: "k_pathPool<DECOMPOSITION_TRACKING, NanoAccessT<false, false>, false, true>"}
+
+
+def path_kernels(mode: str, grid: str, drain: bool) -> str:
+    """The kernels of one launch, whose time is its launch_ms: the pool and, where its last paths are left to it, the
+    drain."""
+    pool = f"k_pathPool<{mode}, {grid}, false, {str(drain).lower()}>"
+    return f"{pool} + k_pathDrain<{mode}, {grid}>" if drain else pool
+
+
+# (residual ratio tracking: the launches of this workload are above 2^23 paths)
+MODE_KERNELS = {0: path_kernels("DELTA_TRACKING", "NanoAccessT<false, false>", True),
+                2: path_kernels("RATIO_TRACKING", "NanoAccessT<false, false>", True),
+                4: path_kernels("RESIDUAL_RATIO_TRACKING", "NanoAccessT<false, false>", False),
+                3: path_kernels("DECOMPOSITION_TRACKING", "NanoAccessT<false, false>", True)}
 
 
 def setup_c1(vpt, torch):
@@ -620,7 +631,7 @@ def run_c5(args, vpt, torch):
                              "denoised_8spp": [round(p["denoised_rel_mse"], 6) for p in per]},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": load_traffic("c5_fp16_2048"),
-                     "kernel": "k_pathPool<RESIDUAL_RATIO_TRACKING, NanoAccessT<false, false>, false, false>", "launches_per_frame": launches,
+                     "kernel": MODE_KERNELS[4], "launches_per_frame": launches,
                      "launch_ms": round(kernel_ms / launches, 3), "algorithmic_bytes_per_launch": int(b_alg / launches),
                      "counters_per_frame": {k: int(v) for k, v in c.items()}},
         "cpu_baseline": None,
@@ -940,7 +951,7 @@ def main() -> int:
                   "majorant": "16^3 supervoxel grid",
                   "step": "one render of each of the 12 estimator x g combinations (12 x 268,435,456 paths)"}
     else:
-        kernel = "k_pathPool<NEXT_EVENT_TRACKING, DenseAccessT<false>, false, true>"
+        kernel = path_kernels("NEXT_EVENT_TRACKING", "DenseAccessT<false>", True)
         config = {"workload": args.workload, "volume": "dense 128^3 fp32 fBm seed 0", "image": f"{W}x{H}",
                   "spp_per_step": spp, "estimator": "next event tracking", "phase_g": 0.85, "albedo": 0.9,
                   "extinction": 1024.0, "environment": "constant white image + directional sun",

@@ -25,7 +25,8 @@ constexpr size_t kFragBytes = size_t(kKpnLayers) * 9 * 2 * 64 * 16;  // bf16x8 f
 
 // Persistent convolution workgroups per CU: the two that fit (148 vector registers and 32 accumulators per lane), so that
 // every tile after a workgroup's first has its halo prefetched and the weights are read once (1920x1080 inference with
-// 1 / 2 / 3 / 4 / 8 per CU: 628 / 569 / 614 / 572 / 597 us).
+// 1 / 2 / 3 / 4 / 8 per CU: 471 / 391 / 451 / 404 / 425 us; a training step on 16 crops of 128^2: 377 / 345 / 357 / 360 /
+// 362 us).
 constexpr int kConvBlocksPerCU = 2;
 
 struct KpnModel {

@@ -210,8 +210,9 @@ struct NanoAccessT {
         return lookupWorldJ(P, pos, jx, jy, jz);
     }
 };
-using NanoAccess = NanoAccessT<true>;        // any grid (lookups, tables, transmittance, batched queue)
+using NanoAccess = NanoAccessT<true>;         // any grid (lookups, tables, batched queue)
 using NanoAccessNarrow = NanoAccessT<false>;  // grids below 4 GiB with axis-aligned voxels (single-frame path kernels)
-using NanoAccessNarrowPoint = NanoAccessT<false, false>;  // ... with a point filter
+// ... with a point filter (path kernels, transmittance; transmittance takes NanoAccess for the other grids and filters)
+using NanoAccessNarrowPoint = NanoAccessT<false, false>;
 
 }  // namespace crvpt
