@@ -2123,9 +2123,14 @@ bool sameLaunch(const BatchLaunch& a, const BatchLaunch& b) {
            a.samplesPerUnit == b.samplesPerUnit;
 }
 
-// Units of one sample leave the launch's last paths to the drain (the table of units has been uploaded).
+// Units of one sample leave the launch's last paths to the drain, where the estimator has one.
+bool batchDrains(const Batch& b, const BatchLaunch& c) {
+    return c.samplesPerUnit == 1u && b.mode != VPT_SPECTRAL_DELTA_TRACKING && b.mode != VPT_NEXT_EVENT_TRACKING_SPECTRAL;
+}
+
+// The drain's memory (the table of units has been uploaded).
 int prepareBatchDrain(Batch& b, const BatchLaunch& c) {
-    if (c.samplesPerUnit != 1u) return CRVPT_OK;
+    if (!batchDrains(b, c)) return CRVPT_OK;
     const uint64_t states = batchDrainStates(b.totalUnits, uint64_t(c.numBlocks) * uint64_t(c.blockSize));
     HIP_TRY(b.dDrain.ensure(std::max<uint64_t>(states, 1) * kDrainWords * sizeof(uint32_t)));
     return CRVPT_OK;
@@ -2135,7 +2140,7 @@ hipError_t enqueueBatch(Batch& b, const BatchLaunch& c, hipStream_t s) {
     return launchBatch(b.mode, b.dReqs.as<BatchRequest>(), b.dUnitBegins.as<uint64_t>(), b.dPixBegins.as<uint64_t>(),
                        int(b.reqs.size()), b.totalUnits, b.totalPix, c, b.dFrame.as<uint32_t>(),
                        b.dRecords.as<float4>(), b.dCounter.as<uint32_t>(),
-                       c.samplesPerUnit == 1u ? b.dDrain.as<uint32_t>() : nullptr, uint32_t(g_r->cuCount) * 4u, s);
+                       batchDrains(b, c) ? b.dDrain.as<uint32_t>() : nullptr, uint32_t(g_r->cuCount) * 4u, s);
 }
 
 bool validBatchLaunch(const BatchLaunch& c) {

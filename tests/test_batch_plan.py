@@ -79,3 +79,26 @@ def test_many_workgroups_take_little_memory(vpt):
         assert blocks == 0 or used < 64 << 20, f"{blocks} workgroups: {used >> 20} MiB"
     assert torch.equal(images[0], images[1])
     vpt.batch_clear()
+
+
+@pytest.mark.gpu
+def test_spectral_batches_take_no_drain(vpt):
+    """2^20 paths of an estimator without a drain: 16 MiB of unit records, and no states beside them (30 MiB and more)."""
+    import torch
+
+    print("case: batch memory of spectral delta tracking", flush=True)
+    vpt.generate_fbm_cloud(20, 20, 20, seed=9)
+    vpt.set_use_sparse_grid(False)
+    vpt.set_vpt_mode(1)
+    vpt.set_extinction_scale(50.0)
+    for side in (16, 512):
+        vpt.batch_clear()
+        vpt.batch_add_request(torch.zeros((3, side, side), dtype=torch.float32, device="cuda"), 4)
+        vpt.batch_set_launch_config(0, 256, 8, 1)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        vpt.batch_render()
+        torch.cuda.synchronize()
+        used = free - torch.cuda.mem_get_info()[0]
+    assert used < 24 << 20, f"{used >> 20} MiB"
+    vpt.batch_clear()
