@@ -25,10 +25,10 @@ namespace crvpt {
 struct BatchGrid {
     const BatchRequest* R;
     using Cache = LeafCache;
-    template <bool FUSE_YZ>
+    template <class TAP>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, LeafCache& c) const {
         if (R->P.sparse) return NanoAccess{R->nano}.lookupWorldJ(P, pos, jx, jy, jz, c);
-        return DenseAccess{R->dense}.lookupWorldJ<FUSE_YZ>(P, pos, jx, jy, jz);
+        return DenseAccess{R->dense}.lookupWorldJ<TAP>(P, pos, jx, jy, jz);
     }
 };
 // Batches write no feature maps.

@@ -339,21 +339,25 @@ struct DenseAccessT {
         const V3 u = plainAdd(v3(0.0f, d.y * P.worldToTex[1], d.z * P.worldToTex[2]), v3(0.0f, jy, jz));
         return v3(x, u.y, u.z);
     }
-    // The tap of the path trackers. FUSE_YZ (fusedTap): the rounding of the point filter's texel coordinate. It is
+    // The tap of the path trackers. TAP::kFuseYZ (PathTap): the rounding of the point filter's texel coordinate. It is
     // written out because a path may be traced in several kernels (pool, start, drain), which hand it over at a time
     // that depends on the schedule: left to the compiler, one kernel fused this sum and another did not, and about one
-    // path in 10^6 read another voxel in the drain than it would have read in the pool.
-    template <bool FUSE_YZ>
+    // path in 10^6 read another voxel in the drain than it would have read in the pool. TAP::kSelectJitter: the other
+    // point filter's coordinate by a jitter of 0 (the same value), not by a choice between the two coordinates.
+    template <class TAP>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz) const {
         if (TRI) return lookupTex(P, toTex(P, pos), jx, jy, jz);
-        // (a jitter of 0 leaves the product of the other filters as it is)
         const bool jitter = P.interpolation == INTERP_STOCHASTIC;
-        const V3 u = toTexJ<FUSE_YZ>(P, pos, jitter ? jx : 0.0f, jitter ? jy : 0.0f, jitter ? jz : 0.0f);
+        V3 u;
+        if constexpr (TAP::kSelectJitter)
+            u = toTexJ<TAP::kFuseYZ>(P, pos, jitter ? jx : 0.0f, jitter ? jy : 0.0f, jitter ? jz : 0.0f);
+        else
+            u = jitter ? toTexJ<TAP::kFuseYZ>(P, pos, jx, jy, jz) : toTex(P, pos);
         return voxel(int(floorf(u.x)), int(floorf(u.y)), int(floorf(u.z)));
     }
-    template <bool FUSE_YZ>
+    template <class TAP>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, NoCache&) const {
-        return lookupWorldJ<FUSE_YZ>(P, pos, jx, jy, jz);
+        return lookupWorldJ<TAP>(P, pos, jx, jy, jz);
     }
     CRVPT_DEV float lookupWorld(const SceneParams& P, Rng& rng, V3 pos) const {
         float jx = 0.0f, jy = 0.0f, jz = 0.0f;

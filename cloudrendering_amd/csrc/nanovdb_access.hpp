@@ -186,8 +186,8 @@ struct NanoAccessT {
         LeafCache c;
         return lookupWorldJ(P, pos, jx, jy, jz, c);
     }
-    // The path trackers' form: the rounding choice concerns dense grids only (DenseAccessT::lookupWorldJ).
-    template <bool FUSE_YZ>
+    // The path trackers' form: the choices of TAP concern dense grids only (DenseAccessT::lookupWorldJ).
+    template <class TAP>
     CRVPT_DEV float lookupWorldJ(const SceneParams& P, V3 pos, float jx, float jy, float jz, LeafCache& cache) const {
         return lookupWorldJ(P, pos, jx, jy, jz, cache);
     }
