@@ -154,7 +154,7 @@ __device__ __forceinline__ void loadBias(const float* __restrict__ bias, int kb,
 }
 
 // Stores the wave's four output rows from row y on, pixel column x, with the layer's epilogue (k_conv3x3): a lane's
-// eight channels in one 16-byte store (two for f32), so a wave writes whole lines (as two 8-byte stores per lane, each
+// eight channels in one 16-byte store, so a wave writes whole lines (as two 8-byte stores per lane, each
 // instruction half of every pixel, a hidden layer took 57 us at 1920x1080 instead of 55).
 template <int EPI>
 __device__ __forceinline__ void storeTile(const f32x4 (&acc)[4][2], const float (&bco)[2][4],
